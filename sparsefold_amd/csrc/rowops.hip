@@ -313,7 +313,9 @@ __device__ __forceinline__ void linear_rows(const sf_linear_args& a, float* ct, 
 // Linear, K % 64 == 0: BMxBN tile, 4 waves (2x2), K in steps of 64 double-buffered in LDS
 // through direct-to-LDS loads (global_load_lds_dwordx4: lane L fills bytes 16L..16L+15 of a
 // 1 KB chunk = 8 rows x 64 k).  Rows are 128 bytes with their 16-byte slots XOR-swizzled by
-// (row & 7), so the operand reads of 8 consecutive lanes hit 8 distinct slots.  The product is
+// (row / 2) % 8, so that the 16 rows whose operand reads are served together (two to each 256-byte
+// span of the 64 banks) hit 16 distinct slots: swizzled by row % 8, rows r and r + 8 met in one
+// bank group and the reads ran at half rate (122 against 235 bytes a clock per CU).  The product is
 // formed transposed (A operand = weight rows), so each lane owns one output row and 4
 // consecutive columns per register group: 8-byte epilogue loads and stores.
 // ------------------------------------------------------------------------------------
@@ -350,7 +352,6 @@ __global__ __launch_bounds__(256) void linear64_kernel(const sf_linear_args a) {
   const int64_t bz = (int64_t)bzu;                            // batch member (0 unless batched)
   const uint16_t* xp = (const uint16_t*)a.x + bz * a.x_bs;
   const uint16_t* wp = (const uint16_t*)a.wt + bz * a.w_bs;
-  const int rsw = 8 * ((lane & 7) ^ ((lane >> 3) & 7));       // this lane's swizzled source piece
   const int64_t mlast = a.M - 1;
   const int nlast = a.N - 1;
 
@@ -358,6 +359,7 @@ __global__ __launch_bounds__(256) void linear64_kernel(const sf_linear_args a) {
 #pragma unroll
     for (int u = 0; u < CPW; ++u) {
       const int c = wave * CPW + u;                            // uniform
+      const int rsw = 8 * ((lane & 7) ^ (4 * (c & 1) + (lane >> 4)));   // this lane's swizzled source piece
       const uint16_t* src;
       if (c < ABYTES / 1024) {
         const int64_t row = min(m0 + c * 8 + (lane >> 3), mlast);
@@ -370,7 +372,7 @@ __global__ __launch_bounds__(256) void linear64_kernel(const sf_linear_args a) {
     }
   };
   auto slot = [&](int buf, int region, int row, int piece) __attribute__((always_inline)) -> const uint8_t* {
-    return smem + buf * BUF + region + (row * 8 + (piece ^ (row & 7))) * 16;
+    return smem + buf * BUF + region + (row * 8 + (piece ^ ((row >> 1) & 7))) * 16;
   };
 
   f32x16 acc[MB][NB];
@@ -780,6 +782,7 @@ extern "C" int sf_hip_linear_fwd(const sf_linear_args* a, void* stream) {
   }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (a->K % 64 == 0) {
+    if (sf_linear_pp_ok(a)) return sf_linear_pp_launch(a, st);
     // largest tile that still gives >= 512 workgroups (two per CU); else the smallest
     auto tiles = [&](int bm, int bn) { return ((a->M + bm - 1) / bm) * (int64_t)((a->N + bn - 1) / bn) * batch; };
     int bm = 64, bn = 64;

@@ -147,6 +147,10 @@ int sf_resident_workgroups(const void* kernel, int threads);
 // split their key range into slices merged by a combine kernel.
 size_t sf_attention_workspace_bytes(const sf_attention_args* a);
 int sf_attention_run(const sf_attention_args* a, void* workspace, size_t workspace_bytes, hipStream_t stream);
+// Linear on large grids (256 x 256 tiles): whether it serves `a` (checked as sf_hip_linear_fwd does
+// before it asks), and its launch.
+bool sf_linear_pp_ok(const sf_linear_args* a);
+int sf_linear_pp_launch(const sf_linear_args* a, hipStream_t stream);
 // Shared-bias attention (5 samples, head dim 48, one bias for every sample): whether it serves
 // `a` (else *why names the first condition that fails), and its launch.
 bool sf_sb_attention_ok(const sf_attention_args* a, const char** why);

@@ -34,8 +34,9 @@ constexpr int kTP = 34;            // LDS pitch of a staged [128 channels][32 po
 static_assert(kC * kTP == 32 * kWS, "the staged product block fills a wave's output rows exactly");
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
-int64_t plane_stride(int N) { return ((int64_t)N * N + 31) & ~(int64_t)31; }
 int padded_n(int N) { return (N + 63) & ~63; }
+// product planes: N rows of Pn columns, so that every row starts on a 128-byte line whatever N is
+int64_t plane_stride(int N) { return (int64_t)N * padded_n(N); }
 
 // Folded weights and offsets, one block of rows each: GLU (left_norm), output (center_norm),
 // gate (left_norm).
@@ -177,8 +178,9 @@ __global__ __launch_bounds__(64 * kTW) void trimul_proj_kernel(const ProjArgs a)
 }
 
 struct OutArgs {
-  int64_t P, Pp;
-  const uint16_t* t;             // [128][Pp] channel-major product
+  int N, Pn, cbs;                // cbs = ceil(N / 32) column blocks per row
+  int64_t Pp;                    // plane stride, N * Pn
+  const uint16_t* t;             // [128][N][Pn] channel-major product
   const uint16_t* z;             // [P, 128]
   const uint16_t* wo;            // folded output projection [128 out, 128 in]
   const float* oo;               // [128]
@@ -186,7 +188,7 @@ struct OutArgs {
   const float* og;               // [128]
   int add_residual;
   uint16_t* out;                 // [P, 128]
-  int items, items_per_wave;
+  int items, items_per_wave;     // 32-column blocks of one row: N * cbs
 };
 
 // D^T = W X^T per 32 output channels x 32 positions: lane (li, half) ends with position li at
@@ -224,16 +226,17 @@ __global__ __launch_bounds__(64 * kTW) void trimul_out_kernel(const OutArgs a) {
   for (int k = 0; k < a.items_per_wave; ++k) {
     const int item = base + k * kTW + wave;
     if (item >= a.items) break;
-    const int64_t p = (int64_t)item * 32 + li;
-    const bool ok = p < a.P;
+    const int row = item / a.cbs, j0 = 32 * (item - row * a.cbs);
+    const bool ok = j0 + li < a.N;
+    const int64_t p0 = (int64_t)row * a.N + j0, p = p0 + li;   // position of column j0, of this lane's column
     // the block's product, [128 channels][32 positions] (64 contiguous bytes per channel): 16-byte
     // loads into the wave's LDS rows at pitch 34, then each lane reads channels 16 kk + 8 half + 0..7
-    // of its position.  Positions past P read the planes' padding (Pp >= item * 32 + 32).
+    // of its position.  Columns past N read the row's padding (j0 + 32 <= Pn).
     u32x4 tv[8], zn[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int q = lane + 64 * u, c = q >> 2, seg = q & 3;
-      tv[u] = ld16(a.t + (int64_t)c * a.Pp + (int64_t)item * 32 + 8 * seg);
+      tv[u] = ld16(a.t + (int64_t)c * a.Pp + (int64_t)row * a.Pn + j0 + 8 * seg);
     }
     const uint16_t* zp = a.z + (ok ? p : 0) * kC + 8 * half;
 #pragma unroll
@@ -306,9 +309,8 @@ __global__ __launch_bounds__(64 * kTW) void trimul_out_kernel(const OutArgs a) {
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int q = lane + 64 * u, pos = q >> 4, c8 = (q & 15) * 8;
-      const int64_t pp = (int64_t)item * 32 + pos;
       const u32x4 v = ld16(&rows[pos * kWS + c8]);
-      if (pp < a.P) st16(a.out + pp * kC + c8, v);
+      if (j0 + pos < a.N) st16(a.out + (p0 + pos) * kC + c8, v);
     }
     asm volatile("" ::: "memory");                    // one wave's LDS accesses run in order
   }
@@ -326,7 +328,7 @@ Ws carve(char* base, int N) {
   size_t off = 0;
   auto take = [&](size_t bytes) { char* p = base ? base + off : nullptr; off += align256(bytes); return p; };
   const size_t ab = (size_t)padded_n(N) * padded_n(N) * kC * 2;      // a / b planes, [c][Pn][Pn]
-  const size_t tp = (size_t)plane_stride(N) * kC * 2;                 // t planes, [c][Pp]
+  const size_t tp = (size_t)plane_stride(N) * kC * 2;                 // t planes, [c][N][Pn]
   w.wglu = reinterpret_cast<uint16_t*>(take((size_t)kGlu * kC * 2));
   w.wout = reinterpret_cast<uint16_t*>(take((size_t)kC * kC * 2));
   w.wgate = reinterpret_cast<uint16_t*>(take((size_t)kC * kC * 2));
@@ -381,7 +383,7 @@ extern "C" int sf_hip_triangle_mult_fwd(const sf_triangle_mult_args* a, void* wo
   }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const int N = a->N, Pn = padded_n(N);
-  const int64_t P = (int64_t)N * N, Pp = plane_stride(N);
+  const int64_t Pp = plane_stride(N);
   const Ws w = carve(static_cast<char*>(workspace), N);
 
   FoldArgs f{};
@@ -408,21 +410,22 @@ extern "C" int sf_hip_triangle_mult_fwd(const sf_triangle_mult_args* a, void* wo
     if ((rc = sf_check_launch("trimul_proj_kernel"))) return rc;
   }
 
-  // t[c][i][j] = sum_k A[c][i][k] B[c][j][k], rows i, j < N, contraction over the padded Pn
+  // t[c][i][j] = sum_k A[c][i][k] B[c][j][k], rows i < N, columns j < Pn (those past N are sums of the
+  // planes' zero rows), contraction over the padded Pn
   {
     sf_linear_args g{};
-    g.M = N; g.N = N; g.K = Pn;
+    g.M = N; g.N = Pn; g.K = Pn;
     g.x = a->incoming ? w.b : w.a; g.x_rs = Pn;
     g.wt = a->incoming ? w.a : w.b;
     g.mul_rows = 1;
-    g.y = w.t; g.y_rs = N;
+    g.y = w.t; g.y_rs = Pn;
     g.batch = kC; g.x_bs = (int64_t)Pn * Pn; g.w_bs = (int64_t)Pn * Pn; g.y_bs = Pp;
     if ((rc = sf_hip_linear_fwd(&g, st))) return rc;
   }
 
-  const int items = (int)((P + 31) / 32);              // 32-position blocks of the output
+  const int cbs = (N + 31) / 32, items = N * cbs;      // 32-column blocks of the output rows
   OutArgs oa{};
-  oa.P = P; oa.Pp = Pp; oa.t = w.t; oa.z = static_cast<const uint16_t*>(a->z);
+  oa.N = N; oa.Pn = Pn; oa.cbs = cbs; oa.Pp = Pp; oa.t = w.t; oa.z = static_cast<const uint16_t*>(a->z);
   oa.wo = w.wout; oa.oo = w.oout; oa.wg = w.wgate; oa.og = w.ogate;
   oa.add_residual = a->add_residual; oa.out = static_cast<uint16_t*>(a->out); oa.items = items;
   const int waves = launch_grid(reinterpret_cast<const void*>(trimul_out_kernel), items);

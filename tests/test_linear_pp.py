@@ -1,0 +1,143 @@
+"""The 256 x 256-tile GEMM behind sf_hip_linear_fwd (csrc/linear_pp.hip).
+
+CPU: its tile order, the LDS layout of a step (what the copies write against what the operand
+reads fetch) and the epilogue's private block, restated from the kernel.  GPU: parity with an fp32
+product at the edges of its tiles and of its K steps, every epilogue, and the calls that must stay
+on the general kernels (an update in place)."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+TILE, BAND = 256, 5
+
+
+@pytest.mark.parametrize("gx,gy,batch", [(1, 1, 1), (20, 12, 1), (15, 12, 1), (16, 13, 1), (20, 17, 1), (3, 3, 128), (2, 2, 128), (7, 1, 9)])
+def test_every_tile_is_taken_once(gx, gy, batch):
+  total = gx * gy * batch
+  t = np.arange(total)
+  bz = t // (gx * gy)
+  r = t - bz * gx * gy
+  band = r // (BAND * gy)
+  q = r - band * BAND * gy
+  bh = np.minimum(BAND, gx - band * BAND)
+  by = q // bh
+  bx = band * BAND + q - by * bh
+  assert (bx >= 0).all() and (bx < gx).all() and (by < gy).all() and (bz < batch).all()
+  assert np.unique(bx + gx * (by + gy * bz)).size == total
+  # the workgroups' walks: XCD ranges of ceil(total / 8), each dealt over the XCD's workgroups
+  grid = min(256, (total + 7) // 8 * 8)
+  per, seen = (total + 7) // 8, np.zeros(total, int)
+  for b in range(grid):
+    tile, end = (b & 7) * per + (b >> 3), min(total, ((b & 7) + 1) * per)
+    while tile < end:
+      seen[tile] += 1
+      tile += grid >> 3
+  assert (seen == 1).all()
+
+
+def test_step_layout_and_bank_groups():
+  """A chunk's lanes write (row, piece) where the operand reads of that row and piece look, and the 16
+  lanes served together read 16 different 16-byte columns of the 256-byte bank span."""
+  lane = np.arange(64)
+  crow, cpiece = lane >> 2, (lane & 3) ^ ((lane >> 4) & 3)
+  where = {}
+  for chunk in range(TILE // 16):
+    for l in range(64):
+      where[(16 * chunk + crow[l], cpiece[l])] = chunk * 1024 + 16 * l
+  half, li = lane >> 5, lane & 31
+  for block in range(TILE // 32):
+    for kk in range(2):
+      addr = (block * 2048 + li * 64 + (half ^ ((li >> 2) & 3)) * 16) ^ (32 * kk)
+      for l in range(64):
+        assert addr[l] == where[(32 * block + li[l], 2 * kk + half[l])]
+      for g in range(4):
+        assert np.unique(addr[16 * g:16 * g + 16] % 256).size == 16
+
+
+@pytest.mark.parametrize("rb", [128, 64])
+def test_epilogue_block_is_a_permutation(rb):
+  row, piece = np.meshgrid(np.arange(32), np.arange(rb // 16), indexing="ij")
+  slot = row * rb + ((piece ^ ((row * rb >> 8) & (rb // 16 - 1))) << 4)
+  assert np.array_equal(np.sort(slot.ravel()), np.arange(32 * rb // 16) * 16)
+
+
+def _check(y, ref, what):
+  """bf16 rounding of the result (2^-8 of its value, half a step and the sum's fp32 error with it)."""
+  err = (y.float() - ref).abs()
+  bound = ref.abs() * 2.0 ** -8 + 1e-3 * ref.square().mean().sqrt()
+  assert bool((err <= bound).all()), f"{what}: {int((err > bound).sum())} values off, worst {float((err - bound).max()):.3e}"
+
+
+def _inputs(M, N, K, seed=3):
+  g = torch.Generator(device="cuda").manual_seed(seed)
+  r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+  return (r(M, K).bfloat16(), (r(N, K) / K ** 0.5).bfloat16(), r(N), r(M, N).bfloat16(), r(96, N).bfloat16())
+
+
+# whole tiles; remainders of rows and columns (8 the smallest); the fewest K steps; several tiles to
+# a workgroup, the last round partly filled
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(5120, 3072, 768), (3850, 3080, 192), (5000, 4104, 128), (6400, 6152, 448), (4097, 3576, 256)])
+@pytest.mark.parametrize("epilogue", ["plain", "bias", "sigmoid_mul", "mul_residual", "glu"])
+def test_parity(M, N, K, epilogue):
+  from sparsefold_amd import _lib
+  from sparsefold_amd.backends.hip import ops
+  x, w, b, res, mul = _inputs(M, N, K)
+  ref = x.float() @ w.float().t()
+  if epilogue == "plain":
+    _check(ops.linear(x, w), ref, epilogue)
+  elif epilogue == "bias":
+    _check(ops.linear(x, w, b), ref + b, epilogue)
+  elif epilogue == "sigmoid_mul":
+    rows = torch.arange(M, device="cuda") % 96
+    _check(ops.linear(x, w, b, post_sigmoid=True, mul=mul), torch.sigmoid(ref + b) * mul.float()[rows], epilogue)
+  elif epilogue == "mul_residual":
+    rows = torch.arange(M, device="cuda") % 96
+    _check(ops.linear(x, w, mul=mul, residual=res), ref * mul.float()[rows] + res.float(), epilogue)
+  else:
+    n = N // 16 * 16
+    y = torch.empty(M, n // 2, dtype=torch.bfloat16, device="cuda")
+    a = _lib.LinearArgs()
+    a.M, a.N, a.K, a.mul_rows, a.glu = M, n, K, 1, 1
+    a.x, a.x_rs, a.wt = x.data_ptr(), K, w.data_ptr()
+    a.y, a.y_rs = y.data_ptr(), n // 2
+    _lib.check(_lib.load().sf_hip_linear_fwd(ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "linear")
+    h = ref[:, :n]
+    _check(y, torch.nn.functional.silu(h[:, 0::2]) * h[:, 1::2], epilogue)
+
+
+@pytest.mark.gpu
+def test_update_in_place_adds_its_residual_once():
+  from sparsefold_amd import _lib
+  M, N, K = 3850, 3080, 192
+  x, w, _, res, _ = _inputs(M, N, K)
+  ref = x.float() @ w.float().t() + res.float()
+  a = _lib.LinearArgs()
+  a.M, a.N, a.K, a.mul_rows = M, N, K, 1
+  a.x, a.x_rs, a.wt = x.data_ptr(), K, w.data_ptr()
+  a.y, a.y_rs, a.residual, a.r_rs = res.data_ptr(), N, res.data_ptr(), N
+  _lib.check(_lib.load().sf_hip_linear_fwd(ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "linear")
+  _check(res, ref, "in place")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [300, 436, 511, 768])
+def test_products_of_the_triangle_multiplication(N):
+  """The batched form (a plane per channel, several tiles to a workgroup), sizes whose rows are not a
+  whole number of pieces, against the 64-bit update."""
+  from oracle import modules as OM
+  from sparsefold_amd import workloads as W
+  from sparsefold_amd import modules as M
+  from sparsefold_amd.backends.hip import modules as HM
+  mod, z, mask = W.make_trimul(N, padded=True, incoming=bool(N % 2), seed=N)
+  hip = HM.TriangleMultiplicationHip(mod.config, M.GlobalConfig(), num_channels=128)
+  hip.load_state_dict(mod.state_dict())
+  hip = hip.cuda()
+  hip.prepare_native()
+  out = hip(z.cuda(), mask.cuda())
+  p = {k: v.cuda().bfloat16().float() if v.ndim == 2 else v.cuda() for k, v in mod.state_dict().items()}
+  ref = OM.triangle_multiplication(z.cuda().float(), mask.cuda(), p, equation=mod.equation)
+  rel = ((out.float() - ref).norm() / ref.norm()).item()
+  assert rel <= 1e-2, rel
