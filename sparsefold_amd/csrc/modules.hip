@@ -1091,6 +1091,7 @@ extern "C" int sf_hip_transition_fwd(const sf_transition_args* a, void* workspac
     return 1;
   }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (sf_transition128_ok(a)) return sf_transition128_launch(a, st);   // one kernel, no workspace
   Arena ws{static_cast<char*>(workspace)};
   const int64_t rows = (int64_t)a->S * a->N;
   int rc;
