@@ -250,14 +250,33 @@ struct Attn2Tile {
   __device__ static int vswz(int key) { return DP == 32 ? 0 : (key >> 1) & 1; }
 };
 
-// KC: 16-dim chunks of q.k that hold data (ceil(D / 16)).  BL: the bias tile goes through LDS
+// Bias rows start where the caller's strides put them (N = 741: at any even address), so bias loads
+// state 2-byte alignment: the global loads are the same instructions, split by the memory unit where
+// a piece crosses a line.
+typedef u32x2 u32x2_any __attribute__((aligned(2)));
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+
+// Elements s .. 7 of the 8 in w moved to 0 .. 7 - s, zeros above (0 < s < 8).
+__device__ __forceinline__ u32x4 shift_down8(u32x4 w, int s) {
+  const int d = s >> 1;                                      // whole words, then a half word
+  u32x4 r = w;
+  if (d & 1) r = u32x4{r[1], r[2], r[3], 0};
+  if (d & 2) r = u32x4{r[2], r[3], 0, 0};
+  if (s & 1) r = u32x4{(r[0] >> 16) | (r[1] << 16), (r[1] >> 16) | (r[2] << 16), (r[2] >> 16) | (r[3] << 16), r[3] >> 16};
+  return r;
+}
+
+// KC: 16-dim chunks of q.k that hold data (ceil(D / 16)).  BL = 1: the bias tile goes through LDS
 // (rows 16-byte aligned, K % 8 == 0): each wave copies its 32 query rows x 64 keys with four
 // direct-to-LDS loads of 8 rows x 128 bytes, slot-major [row/8][piece][row%8], and every lane
 // then reads its keys with conflict-free 8-byte LDS reads.  Loaded lane by lane from global
 // memory instead, every bias instruction touched 32 rows: 40% of the kernel's time.  One buffer
 // per wave: the wave reads the tile's bias into registers first, waits for those reads, and only
 // then copies the next tile's into the same buffer (48 KB per shared-tile workgroup, three per CU).
-template <int DP, bool SHARED, int KC, bool BL>
+// BL = 2: the same tile and layout for rows of any alignment and any K >= 8, loaded 16 bytes a lane
+// into registers a tile ahead (direct-to-LDS copies need aligned rows) and written to LDS at the
+// tile's start.  BL = 0: each lane loads its keys from global memory.
+template <int DP, bool SHARED, int KC, int BL>
 __global__ __launch_bounds__(256) void attn2_kernel(const sf_attention_args a, const Attn2Plan pl) {
   using T = Attn2Tile<DP>;
   constexpr int kWaveBufs = SHARED ? 1 : 4;                 // tile sets in LDS (shared or per wave)
@@ -387,7 +406,28 @@ __global__ __launch_bounds__(256) void attn2_kernel(const sf_attention_args a, c
     brs8 = 8 * a.bias_s[3];
   }
   const bool brows_clamped = qblk * 32 + 32 > Q;            // uniform: the last query block
+  u32x4 breg[4];                                             // BL = 2: the next tile's pieces
   auto load_bias_lds = [&](int j0) __attribute__((always_inline)) {
+    if constexpr (BL == 2) {
+      const int j = j0 + 8 * bpiece, over = max(0, j + 8 - K);   // elements of the piece past the row's end
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint16_t* src = brow0 + u * brs8;
+        if (brows_clamped) {
+          const uint16_t* bh = (const uint16_t*)a.bias + b0 * a.bias_s[0] + b1 * a.bias_s[1] + (int64_t)h * a.bias_s[2];
+          src = bh + (int64_t)min(qblk * 32 + 8 * u + (lane >> 3), Q - 1) * a.bias_s[3] + 8 * bpiece;
+        }
+        breg[u] = *reinterpret_cast<const u32x4_any*>(src + j0 - over);   // the row's last 8 where it ends
+      }
+      if (j0 + 64 > K) {                                     // uniform: the last tile (zeros past the end)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const u32x4 sh = shift_down8(breg[u], over & 7);
+          if (over > 0) breg[u] = over < 8 ? sh : u32x4{0, 0, 0, 0};
+        }
+      }
+      return;
+    }
     const int jc = min(j0, K - 8 - 8 * bpiece) - j0;         // pieces past K re-read the last one
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -407,7 +447,7 @@ __global__ __launch_bounds__(256) void attn2_kernel(const sf_attention_args a, c
     } else if (j0 + 64 <= K) {                               // uniform: the whole tile is in range
 #pragma unroll
       for (int q = 0; q < 8; ++q)                            // keys j0 + 32(q/4) + 8(q%4) + 4half .. +3
-        bnext[q] = *reinterpret_cast<const u32x2*>(bp + j0 + 32 * (q >> 2) + 8 * (q & 3) + 4 * half);
+        bnext[q] = *reinterpret_cast<const u32x2_any*>(bp + j0 + 32 * (q >> 2) + 8 * (q & 3) + 4 * half);
     } else {                                                 // last tile: ragged end of the keys
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
@@ -450,6 +490,11 @@ __global__ __launch_bounds__(256) void attn2_kernel(const sf_attention_args a, c
     const uint8_t* kt = wsm + buf * T::kBufBytes;
     const uint8_t* vt = kt + T::kKBytes;
     u32x2 bcur[8];
+    if constexpr (BL == 2) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) st16(bsm + u * 1024 + lane * 16, breg[u]);
+      asm volatile("" ::: "memory");                         // one wave's LDS accesses run in order
+    }
     if (BL) {                                                // keys 32(q/4) + 8(q%4) + 4half .. +3 = piece q
 #pragma unroll
       for (int q = 0; q < 8; ++q)                            // row li: slot 8 (li%8) + (q ^ li%8) of chunk li/8
@@ -694,8 +739,8 @@ bool aligned8(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7) == 0;
 namespace {
 
 struct AttnRoute {
-  bool vec, vec_out, attn2, shared, bl;
-  int dmax, kc, ksplit;
+  bool vec, vec_out, attn2, shared;
+  int bl, dmax, kc, ksplit;
   Attn2Plan pl;
 };
 
@@ -720,14 +765,11 @@ int route(const sf_attention_args* a, bool allow_split, AttnRoute& r) {
     r.vec = (a->q_s[s] % 8 == 0) && (a->k_s[s] % 8 == 0) && (a->v_s[s] % 8 == 0);
   r.vec_out = aligned8(a->out);
   for (int s = 0; s < 4 && r.vec_out; ++s) r.vec_out = (a->o_s[s] % 4 == 0);
-  bool bias_vec = a->bias == nullptr || aligned8(a->bias);
-  for (int s = 0; s < 4 && bias_vec && a->bias != nullptr; ++s) bias_vec = a->bias_s[s] % 4 == 0;
-  r.attn2 = r.vec && bias_vec;
+  r.attn2 = r.vec;
   r.ksplit = 1;
   r.pl = Attn2Plan{};
   if (a->kv_index != nullptr && (!r.attn2 || a->kv_zero_row < 0)) {
-    sf_set_error("attention: gathered K/V rows need 16-byte aligned q/k/v rows and strides, an 8-byte aligned "
-                 "bias and kv_zero_row >= 0");
+    sf_set_error("attention: gathered K/V rows need 16-byte aligned q/k/v rows and strides and kv_zero_row >= 0");
     return 1;
   }
   if (!r.attn2) return 0;
@@ -737,7 +779,12 @@ int route(const sf_attention_args* a, bool allow_split, AttnRoute& r) {
   for (int s = 0; s < 4 && pl.vec_out && a->gate != nullptr; ++s) pl.vec_out = a->g_s[s] % 4 == 0;
   const int64_t bh = (int64_t)a->B0 * a->B1 * a->H;
   const int64_t groups = bh * ((pl.QB + 3) / 4);
-  r.shared = a->schedule == 0 ? (a->Q >= 128 && groups >= 512) : a->schedule == 1;
+  // Shared tiles from a quarter (head dims above 32) or half of the CUs on: a private wave copies
+  // every K/V tile for its own 32 queries, and its key-range slices cost a combine.  Diffusion
+  // attention block, us private against shared: 5 x 740 133 / 94, 5 x 512 98 / 76, 5 x 256 66 / 54,
+  // 1 x 740 (96 groups) 68 / 65; single attention with head dim 24, N = 740 (96 groups) 98 / 100,
+  // N = 1024 (128 groups) 142 / 142.
+  r.shared = a->schedule == 0 ? (a->Q >= 128 && groups >= (r.dmax > 32 ? 64 : 128)) : a->schedule == 1;
   // Per-wave tasks on a grid too small for the GPU (single attention: 16 heads x 24 blocks =
   // 384 waves for 1024 SIMDs) split their key range into slices of >= 2 tiles, up to ~2048 waves;
   // a combine kernel merges the slices.  Needs a workspace (module-level entry points).
@@ -754,11 +801,13 @@ int route(const sf_attention_args* a, bool allow_split, AttnRoute& r) {
   const int64_t wgs = r.shared ? pl.tasks : (pl.tasks + 3) / 4;
   pl.xcd_order = a->bias != nullptr && a->bias_s[0] == 0 && a->B0 > 1 && wgs % 8 == 0 && (r.shared || pl.tasks % 4 == 0);
   r.kc = (a->D + 15) / 16;                                  // q.k chunks holding data
-  // LDS bias tiles: always with shared tiles; per-wave tiles from two key tiles on (with one
+  // LDS bias tiles (2: rows of any alignment; a diffusion block of 5 x 741 tokens, whose rows the
+  // aligned copies cannot take, 204 -> 95 us with the shared tiles above): always with shared tiles; per-wave tiles from two key tiles on (with one
   // bias buffer per wave a per-wave-tile workgroup takes 80 KB, two per CU as without the bias
   // tiles: atom windows, K = 128, 34.7 -> 30.5 us; single attention, K = 768, 30 -> 25 us)
-  r.bl = a->bias != nullptr && aligned16(a->bias) && a->K % 8 == 0 && (r.shared || a->K >= 128);
-  for (int s2 = 0; s2 < 4 && r.bl; ++s2) r.bl = a->bias_s[s2] % 8 == 0;
+  bool rows16 = aligned16(a->bias) && a->K % 8 == 0;
+  for (int s2 = 0; s2 < 4 && rows16; ++s2) rows16 = a->bias_s[s2] % 8 == 0;
+  r.bl = a->bias == nullptr || !(r.shared || a->K >= 128) || a->K < 8 ? 0 : rows16 ? 1 : 2;
   return 0;
 }
 
@@ -784,8 +833,9 @@ int launch_attention(const sf_attention_args* a, const AttnRoute& r, float* spli
     using Tt = std::true_type;
     using Ff = std::false_type;
     auto by_bl = [&](auto dp, auto sh, auto kcc) {
-      if (r.bl) launch(dp, sh, kcc, Tt{});
-      else launch(dp, sh, kcc, Ff{});
+      if (r.bl == 1) launch(dp, sh, kcc, std::integral_constant<int, 1>{});
+      else if (r.bl == 2) launch(dp, sh, kcc, std::integral_constant<int, 2>{});
+      else launch(dp, sh, kcc, std::integral_constant<int, 0>{});
     };
     auto by_sh = [&](auto dp, auto kcc) {
       if (r.shared) by_bl(dp, Tt{}, kcc);

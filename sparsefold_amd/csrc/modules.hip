@@ -471,7 +471,8 @@ __global__ __launch_bounds__(512) void adaln2_proj_kernel(const Adaln2Args a) {
 void* const kArenaAligned = reinterpret_cast<void*>(static_cast<uintptr_t>(1) << 20);
 
 // workspace of the self-attention chain (the arena walk below, run without a base)
-size_t self_ws(const sf_self_attention_args* a) {
+// (slices: with the attention's key-range slices, as the entry point with a workspace runs it)
+size_t self_ws(const sf_self_attention_args* a, bool slices = true) {
   Arena ws{nullptr};
   const int64_t rows = (int64_t)a->S * a->N;
   const int HD = a->H * a->D;
@@ -484,7 +485,7 @@ size_t self_ws(const sf_self_attention_args* a) {
   ws.take((size_t)rows * 4 * HD * 2);        // q k v g
   ws.take((size_t)rows * HD * 2);            // o
   const sf_attention_args t = self_attn_args(a, kArenaAligned, kArenaAligned);
-  ws.take(sf_attention_workspace_bytes(&t));  // key-range slices of the attention
+  if (slices) ws.take(sf_attention_workspace_bytes(&t));  // key-range slices of the attention
   if (cond_gemms) ws.take((size_t)a->N * a->C * 2);
   return ws.off;
 }
@@ -526,7 +527,7 @@ extern "C" size_t sf_hip_self_attention_workspace_bytes(const sf_self_attention_
 }
 
 static int self_attention_run(const sf_self_attention_args* a, void* workspace, size_t workspace_bytes,
-                              void* stream) {
+                              void* stream, bool slices = true) {
   if (a == nullptr || a->x == nullptr || a->out == nullptr || a->w_qkvg == nullptr || a->w_t2 == nullptr) {
     sf_set_error("self_attention: x, out, w_qkvg and w_t2 must be non-null"); return 1;
   }
@@ -544,8 +545,8 @@ static int self_attention_run(const sf_self_attention_args* a, void* workspace, 
   if (!pre && a->cond && (a->w_scale == nullptr || a->w_shift == nullptr || a->w_zc == nullptr)) {
     sf_set_error("self_attention: a condition needs w_scale, w_shift and w_zc"); return 1;
   }
-  if (workspace == nullptr || workspace_bytes < self_ws(a)) {
-    sf_set_error("self_attention: workspace of %zu bytes needed, %zu given", self_ws(a), workspace_bytes);
+  if (workspace == nullptr || workspace_bytes < self_ws(a, slices)) {
+    sf_set_error("self_attention: workspace of %zu bytes needed, %zu given", self_ws(a, slices), workspace_bytes);
     return 1;
   }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
@@ -590,8 +591,8 @@ static int self_attention_run(const sf_self_attention_args* a, void* workspace, 
   p.mul_rows = 1; p.y = y; p.y_rs = 4 * HD;
   if ((rc = sf_hip_linear_fwd(&p, st))) return rc;
   const sf_attention_args t = self_attn_args(a, y, o);
-  const size_t split = sf_attention_workspace_bytes(&t);
-  void* split_ws = ws.take(split);
+  const size_t split = slices ? sf_attention_workspace_bytes(&t) : 0;
+  void* split_ws = slices ? ws.take(split) : nullptr;
   if ((rc = sf_attention_run(&t, split_ws, split, st))) return rc;
   return zero_init_out(rows, a->C, HD, o, pre || fused_cond ? nullptr : a->cond, a->N, a->Cs, a->w_zc, a->b_zc,
                        a->w_t2, a->add_residual ? a->x : nullptr, a->out, ws, st,
@@ -643,7 +644,9 @@ int scratch_address(void** addr) {
 
 extern "C" int sf_hip_self_attention_fwd_noalloc(const sf_self_attention_args* a, void* stream) {
   if (a == nullptr) { sf_set_error("self_attention_noalloc: null arguments"); return 1; }
-  const size_t need = self_ws(a);
+  // sizes whose key-range slices do not fit run without them
+  const bool slices = self_ws(a) <= (size_t)SF_HIP_NOALLOC_SCRATCH_BYTES;
+  const size_t need = self_ws(a, slices);
   if (need > (size_t)SF_HIP_NOALLOC_SCRATCH_BYTES) {
     sf_set_error("self_attention_noalloc: these sizes need %zu bytes of scratch; the fixed scratch holds %zu "
                  "(use sf_hip_self_attention_fwd with a workspace)", need, (size_t)SF_HIP_NOALLOC_SCRATCH_BYTES);
@@ -651,7 +654,7 @@ extern "C" int sf_hip_self_attention_fwd_noalloc(const sf_self_attention_args* a
   }
   void* ws = nullptr;
   if (int rc = scratch_address(&ws)) return rc;
-  return self_attention_run(a, ws, SF_HIP_NOALLOC_SCRATCH_BYTES, stream);
+  return self_attention_run(a, ws, SF_HIP_NOALLOC_SCRATCH_BYTES, stream, slices);
 }
 
 extern "C" size_t sf_hip_cross_attention_workspace_bytes(const sf_cross_attention_args* a) {

@@ -577,6 +577,7 @@ bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 // The grid holds only as many workgroups as are resident at once, so all of them sweep one
 // contiguous window of every plane together.
 // ------------------------------------------------------------------------------------
+typedef u32x4 u32x4_any __attribute__((aligned(2)));   // a 16-byte store at any even address
 constexpr int kPLWP = 128 + 8;        // LDS pitch (elements) of folded weight rows
 constexpr int kPL128MaxH = 1024;
 constexpr int kPLWaves = 4;           // waves per workgroup (4 and 8 measure the same)
@@ -584,8 +585,9 @@ constexpr int kPLWaves = 4;           // waves per workgroup (4 and 8 measure th
 
 // HB: 32-plane blocks per tile (NP = 32 HB planes); G2: tiles per workgroup (the normalised z
 // operands are reused for G2 * NP planes; H <= G2 * NP * hgroups, and every tile holds a plane
-// h < H); SEG: segmented output; VEC: 16-byte stores (P and seg multiples of 8, out 16-byte
-// aligned), else 2-byte stores.
+// h < H); SEG: segmented output; VEC: 16-byte stores (P and seg multiples of 8, or one segment of any
+// length >= 8: its planes then start at any even address, which the stores allow), else 2-byte stores.
+// (Single update of 1023 tokens, whose planes are an odd number of elements: 142 -> 136 us.)
 //
 // No wait covers a store: the z loads are unconditional (positions past P read position 0, their
 // operands are zeroed and their planes never stored), the loop is rotated so that the next step's
@@ -683,9 +685,9 @@ __global__ __launch_bounds__(64 * W) void pair_logits128_kernel(const sf_pair_lo
     lds_only_barrier();
     const int64_t p = base * 32 + 8 * ch;     // first of this lane's 8 positions
     if constexpr (VEC) {
-      // the last valid chunk (P is a multiple of 8 and the tile holds a position below P) and the
-      // last valid plane of the tile (it holds one)
-      const int64_t pc = min(p, P - 8);
+      // the last whole chunk of 8 positions, or this tile's first where P ends in its first chunk
+      // (then written only by the tail below), and the last valid plane of the tile (it holds one)
+      const int64_t pc = min(p, max((P & ~7ll) - 8, base * 32));
       const int chc = (int)((pc - base * 32) >> 3);
       const int plmax = H - 1 - h0 - g * NP;
 #pragma unroll
@@ -694,7 +696,15 @@ __global__ __launch_bounds__(64 * W) void pair_logits128_kernel(const sf_pair_lo
         const u32x4 v = ld16(T + pl * TP + 8 * chc);
         const int hh = h0 + g * NP + pl;
         const int64_t blk = hh / grp;
-        st16_stream(out + blk * grp * P + (hh - blk * grp) * seg + pos_off(pc), v);
+        if (SEG) st16_stream(out + blk * grp * P + (hh - blk * grp) * seg + pos_off(pc), v);
+        else if (base * 32 + 8 <= P) __builtin_nontemporal_store(v, reinterpret_cast<u32x4_any*>(out + (int64_t)hh * P + pc));
+      }
+      if (!SEG && (P & 7) != 0 && base * 32 + TPOS >= P) {   // uniform: the last P % 8 positions of every plane
+        const int t0 = (int)((P & ~7ll) - base * 32), nt = (int)(P & 7);
+        for (int e = tid; e < 8 * NP; e += 64 * W) {
+          const int pl = e >> 3, q = e & 7;
+          if (q < nt && pl <= plmax) out[(int64_t)(h0 + g * NP + pl) * P + base * 32 + t0 + q] = T[pl * TP + t0 + q];
+        }
       }
     } else {
 #pragma unroll
@@ -829,7 +839,7 @@ extern "C" int sf_hip_pair_logits_fwd(const sf_pair_logits_args* a, void* stream
     const int g2 = (b.H <= 64 || (b.H - 1) % 128 < 64) ? 1 : 2;
     const int hgroups = (b.H + 32 * hb * g2 - 1) / (32 * hb * g2);
     const bool seg = b.seg != b.P;
-    const bool vec = (b.P % 8 == 0) && (b.seg % 8 == 0) && al16(b.out);
+    const bool vec = seg ? (b.P % 8 == 0) && (b.seg % 8 == 0) && al16(b.out) : b.P >= 8;
     auto launch = [&](auto kernel) {
       // position workers (a multiple of 8): enough for every tile, and no more workgroups than are
       // resident at once

@@ -35,8 +35,10 @@ static_assert(kC * kTP == 32 * kWS, "the staged product block fills a wave's out
 
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 int padded_n(int N) { return (N + 63) & ~63; }
-// product planes: N rows of Pn columns, so that every row starts on a 128-byte line whatever N is
-int64_t plane_stride(int N) { return (int64_t)N * padded_n(N); }
+// product planes: N rows of N rounded up to 8 columns, so that every row starts on a 16-byte piece
+// whatever N is, rounded up to whole blocks of 32
+int64_t product_cols(int N) { return (N + 7) & ~7; }
+int64_t plane_stride(int N) { return (N * product_cols(N) + 31) & ~(int64_t)31; }
 
 // Folded weights and offsets, one block of rows each: GLU (left_norm), output (center_norm),
 // gate (left_norm).
@@ -178,9 +180,9 @@ __global__ __launch_bounds__(64 * kTW) void trimul_proj_kernel(const ProjArgs a)
 }
 
 struct OutArgs {
-  int N, Pn, cbs;                // cbs = ceil(N / 32) column blocks per row
-  int64_t Pp;                    // plane stride, N * Pn
-  const uint16_t* t;             // [128][N][Pn] channel-major product
+  int N, Nt;                     // row length and stride (N rounded up to 8) of the product
+  int64_t P, Pp;                 // N * Nt positions of a plane, and its stride
+  const uint16_t* t;             // [128][Pp] channel-major product, rows of Nt
   const uint16_t* z;             // [P, 128]
   const uint16_t* wo;            // folded output projection [128 out, 128 in]
   const float* oo;               // [128]
@@ -188,7 +190,7 @@ struct OutArgs {
   const float* og;               // [128]
   int add_residual;
   uint16_t* out;                 // [P, 128]
-  int items, items_per_wave;     // 32-column blocks of one row: N * cbs
+  int items, items_per_wave;     // blocks of 32 of the P positions
 };
 
 // D^T = W X^T per 32 output channels x 32 positions: lane (li, half) ends with position li at
@@ -226,21 +228,26 @@ __global__ __launch_bounds__(64 * kTW) void trimul_out_kernel(const OutArgs a) {
   for (int k = 0; k < a.items_per_wave; ++k) {
     const int item = base + k * kTW + wave;
     if (item >= a.items) break;
-    const int row = item / a.cbs, j0 = 32 * (item - row * a.cbs);
-    const bool ok = j0 + li < a.N;
-    const int64_t p0 = (int64_t)row * a.N + j0, p = p0 + li;   // position of column j0, of this lane's column
+    // this lane's position of the product plane (below 2^31: N <= 8192) as one of z and out: the
+    // same where rows are unpadded (N a multiple of 8); -1 past the end and at a padding column
+    int p = item * 32 + li;
+    if (p >= a.P) p = -1;
+    if (a.Nt != a.N && p >= 0) {
+      const int row = p / a.Nt, col = p - row * a.Nt;
+      p = col < a.N ? row * a.N + col : -1;
+    }
     // the block's product, [128 channels][32 positions] (64 contiguous bytes per channel): 16-byte
     // loads into the wave's LDS rows at pitch 34, then each lane reads channels 16 kk + 8 half + 0..7
-    // of its position.  Columns past N read the row's padding (j0 + 32 <= Pn).
+    // of its position.  Positions past P read the plane's padding (Pp >= item * 32 + 32), unused.
     u32x4 tv[8], zn[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int q = lane + 64 * u, c = q >> 2, seg = q & 3;
-      tv[u] = ld16(a.t + (int64_t)c * a.Pp + (int64_t)row * a.Pn + j0 + 8 * seg);
+      const int w = lane + 64 * u, c = w >> 2, seg = w & 3;
+      tv[u] = ld16(a.t + (int64_t)c * a.Pp + (int64_t)item * 32 + 8 * seg);
     }
-    const uint16_t* zp = a.z + (ok ? p : 0) * kC + 8 * half;
+    const uint16_t* zp = a.z + (int64_t)max(p, 0) * kC + 8 * half;
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) zn[kk] = ok ? ld16(zp + 16 * kk) : u32x4{0, 0, 0, 0};
+    for (int kk = 0; kk < 8; ++kk) zn[kk] = p >= 0 ? ld16(zp + 16 * kk) : u32x4{0, 0, 0, 0};
     uint32_t* const rw = reinterpret_cast<uint32_t*>(rows);
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -257,14 +264,14 @@ __global__ __launch_bounds__(64 * kTW) void trimul_out_kernel(const OutArgs a) {
       for (int e = 0; e < 4; ++e) {
         const uint32_t lo = rows[(16 * kk + 8 * half + 2 * e) * kTP + li];
         const uint32_t hi = rows[(16 * kk + 8 * half + 2 * e + 1) * kTP + li];
-        w[e] = ok ? lo | (hi << 16) : 0u;
+        w[e] = p >= 0 ? lo | (hi << 16) : 0u;
       }
       tn[kk] = u32x4{w[0], w[1], w[2], w[3]};
     }
     asm volatile("" ::: "memory");                    // (the rows are rewritten below)
     bf16x8 to[8], zo[8];
-    ln128_operands(tn, ok, to);
-    ln128_operands(zn, ok, zo);
+    ln128_operands(tn, p >= 0, to);
+    ln128_operands(zn, p >= 0, zo);
 #pragma unroll
     for (int nb = 0; nb < kC / 32; ++nb) {
       // residual z of this lane's update channels: channel 32 nb + 8 g + 4 half + e is word
@@ -308,9 +315,10 @@ __global__ __launch_bounds__(64 * kTW) void trimul_out_kernel(const OutArgs a) {
     asm volatile("" ::: "memory");                    // one wave's LDS accesses run in order
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int q = lane + 64 * u, pos = q >> 4, c8 = (q & 15) * 8;
+      const int w = lane + 64 * u, pos = w >> 4, c8 = (w & 15) * 8;
       const u32x4 v = ld16(&rows[pos * kWS + c8]);
-      if (j0 + pos < a.N) st16(a.out + (p0 + pos) * kC + c8, v);
+      const int pp = __shfl(p, pos);                  // lane pos holds the block's position pos
+      if (pp >= 0) st16(a.out + (int64_t)pp * kC + c8, v);
     }
     asm volatile("" ::: "memory");                    // one wave's LDS accesses run in order
   }
@@ -328,7 +336,7 @@ Ws carve(char* base, int N) {
   size_t off = 0;
   auto take = [&](size_t bytes) { char* p = base ? base + off : nullptr; off += align256(bytes); return p; };
   const size_t ab = (size_t)padded_n(N) * padded_n(N) * kC * 2;      // a / b planes, [c][Pn][Pn]
-  const size_t tp = (size_t)plane_stride(N) * kC * 2;                 // t planes, [c][N][Pn]
+  const size_t tp = (size_t)plane_stride(N) * kC * 2;                 // t planes, [c][Pp]
   w.wglu = reinterpret_cast<uint16_t*>(take((size_t)kGlu * kC * 2));
   w.wout = reinterpret_cast<uint16_t*>(take((size_t)kC * kC * 2));
   w.wgate = reinterpret_cast<uint16_t*>(take((size_t)kC * kC * 2));
@@ -383,7 +391,8 @@ extern "C" int sf_hip_triangle_mult_fwd(const sf_triangle_mult_args* a, void* wo
   }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const int N = a->N, Pn = padded_n(N);
-  const int64_t Pp = plane_stride(N);
+  const int Nt = (int)product_cols(N);
+  const int64_t P = (int64_t)N * Nt, Pp = plane_stride(N);
   const Ws w = carve(static_cast<char*>(workspace), N);
 
   FoldArgs f{};
@@ -410,22 +419,22 @@ extern "C" int sf_hip_triangle_mult_fwd(const sf_triangle_mult_args* a, void* wo
     if ((rc = sf_check_launch("trimul_proj_kernel"))) return rc;
   }
 
-  // t[c][i][j] = sum_k A[c][i][k] B[c][j][k], rows i < N, columns j < Pn (those past N are sums of the
-  // planes' zero rows), contraction over the padded Pn
+  // t[c][i][j] = sum_k A[c][i][k] B[c][j][k], rows i < N, columns j < N rounded up to whole 16-byte
+  // pieces (those past N are sums of the planes' zero rows), contraction over the padded Pn
   {
     sf_linear_args g{};
-    g.M = N; g.N = Pn; g.K = Pn;
+    g.M = N; g.N = Nt; g.K = Pn;
     g.x = a->incoming ? w.b : w.a; g.x_rs = Pn;
     g.wt = a->incoming ? w.a : w.b;
     g.mul_rows = 1;
-    g.y = w.t; g.y_rs = Pn;
+    g.y = w.t; g.y_rs = Nt;
     g.batch = kC; g.x_bs = (int64_t)Pn * Pn; g.w_bs = (int64_t)Pn * Pn; g.y_bs = Pp;
     if ((rc = sf_hip_linear_fwd(&g, st))) return rc;
   }
 
-  const int cbs = (N + 31) / 32, items = N * cbs;      // 32-column blocks of the output rows
+  const int items = (int)((P + 31) / 32);              // 32-position blocks of the output
   OutArgs oa{};
-  oa.N = N; oa.Pn = Pn; oa.cbs = cbs; oa.Pp = Pp; oa.t = w.t; oa.z = static_cast<const uint16_t*>(a->z);
+  oa.N = N; oa.Nt = Nt; oa.P = P; oa.Pp = Pp; oa.t = w.t; oa.z = static_cast<const uint16_t*>(a->z);
   oa.wo = w.wout; oa.oo = w.oout; oa.wg = w.wgate; oa.og = w.ogate;
   oa.add_residual = a->add_residual; oa.out = static_cast<uint16_t*>(a->out); oa.items = items;
   const int waves = launch_grid(reinterpret_cast<const void*>(trimul_out_kernel), items);
