@@ -244,6 +244,113 @@ struct TriProjArgs {
   int items, items_per_wave;          // items = NP * NP / 32 position blocks
 };
 
+// One block of 32 folded projection rows (rows 32 nb .. of sW, offsets sOff) of 32 positions p0 + li
+// of attention row r, from the normalised z operands xo.
+//
+// q, k (which = 0, 1): D^T = W . X^T -> lane = position; registers 8*kk .. 8*kk+7 are the 16 bytes
+// of k-chunk kk (KC = 2) or of head 2 hh + kk (KC = 1) in the Q/K layout
+template <int KC>
+__device__ __forceinline__ void proj_qk_block(const TriProjArgs& a, int which, int hh, const uint16_t* sW, const float* sOff,
+                                              int nb, const bf16x8 (&xo)[TriDims<KC>::NC], bool valid, int r, int p, int lane) {
+  constexpr int WP = TriDims<KC>::WP, NC = TriDims<KC>::NC;
+  const int half = lane >> 5, li = lane & 31;
+  uint16_t* dst = which == 0 ? a.q : a.k;
+  const float sc = which == 0 ? a.qscale : 1.0f;
+  f32x16 acc;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+#pragma unroll
+  for (int kk = 0; kk < NC; ++kk)
+    acc = mfma32(as_bf16x8(ld16(&sW[(32 * nb + li) * WP + 16 * kk + 8 * half])), xo[kk], acc);
+  // KC = 2: k-chunk kk of head hh, 512 elements apart; KC = 1: head 2 hh + kk (NP * 16 apart)
+  uint16_t* op = dst + ql_off<KC>(r, KC == 2 ? hh : 2 * hh, a.H, a.NP, p, 0, half);
+  constexpr int kStep = KC == 2 ? 512 : 0;
+  const int64_t step = KC == 2 ? kStep : (int64_t)a.NP * 16;
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk) {
+    const f32x4 o0 = *reinterpret_cast<const f32x4*>(&sOff[32 * nb + 16 * kk + 4 * half]);
+    const f32x4 o1 = *reinterpret_cast<const f32x4*>(&sOff[32 * nb + 16 * kk + 8 + 4 * half]);
+    uint32_t w[4];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      w[e] = pack_bf2(valid ? (acc[8 * kk + 2 * e] + o0[2 * e]) * sc : 0.f,
+                      valid ? (acc[8 * kk + 2 * e + 1] + o0[2 * e + 1]) * sc : 0.f);
+      w[2 + e] = pack_bf2(valid ? (acc[8 * kk + 4 + 2 * e] + o1[2 * e]) * sc : 0.f,
+                          valid ? (acc[8 * kk + 4 + 2 * e + 1] + o1[2 * e + 1]) * sc : 0.f);
+    }
+    st16_stream(op + kk * step, u32x4{w[0], w[1], w[2], w[3]});
+  }
+}
+
+// v: D = X . W^T -> lane = projection row li (head hh, dim li for KC = 2; head 2 hh + li / 16,
+// dim li % 16 for KC = 1); registers 8*cc .. 8*cc+7 are keys of 16-key chunk cc of this block
+// in PV slot order for lane half `half`
+template <int KC>
+__device__ __forceinline__ void proj_v_block(const TriProjArgs& a, int hh, const uint16_t* sW, const float* sOff, int nb,
+                                             const bf16x8 (&xo)[TriDims<KC>::NC], int r, int p0, int lane) {
+  constexpr int WP = TriDims<KC>::WP, NC = TriDims<KC>::NC;
+  const int half = lane >> 5, li = lane & 31;
+  f32x16 acc;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+#pragma unroll
+  for (int kk = 0; kk < NC; ++kk)
+    acc = mfma32(xo[kk], as_bf16x8(ld16(&sW[(32 * nb + li) * WP + 16 * kk + 8 * half])), acc);
+  const float off = sOff[32 * nb + li];
+  const int vh = KC == 2 ? hh : 2 * hh + (li >> 4), vd = KC == 2 ? li : li & 15;
+#pragma unroll
+  for (int cc = 0; cc < 2; ++cc) {
+    uint32_t w[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int t0 = 2 * e, t1 = 2 * e + 1;             // slot t -> key 16cc + 8(t/4) + 4half + t%4
+      const int k0 = p0 + 16 * cc + 8 * (t0 >> 2) + 4 * half + (t0 & 3);
+      const int k1 = p0 + 16 * cc + 8 * (t1 >> 2) + 4 * half + (t1 & 3);
+      w[e] = pack_bf2(r < a.N && k0 < a.N ? acc[8 * cc + t0] + off : 0.f, r < a.N && k1 < a.N ? acc[8 * cc + t1] + off : 0.f);
+    }
+    st16_stream(a.vt + vl_off<KC>(r, vh, a.H, a.NP, (p0 >> 4) + cc, half, vd), u32x4{w[0], w[1], w[2], w[3]});
+  }
+}
+
+// bias planes: D = X . Wb^T, lane = head li (< H), 4 consecutive positions; bit j of mbits = the
+// sequence mask of the key of position p0 + j
+template <int KC>
+__device__ __forceinline__ void proj_bias_block(const TriProjArgs& a, const uint16_t* sW, const float* sOff, int nb,
+                                                const bf16x8 (&xo)[TriDims<KC>::NC], uint32_t mbits, int r, int p0, int lane) {
+  constexpr int WP = TriDims<KC>::WP, NC = TriDims<KC>::NC;
+  const int half = lane >> 5, li = lane & 31;
+  f32x16 acc;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+#pragma unroll
+  for (int kk = 0; kk < NC; ++kk)
+    acc = mfma32(xo[kk], as_bf16x8(ld16(&sW[(32 * nb + li) * WP + 16 * kk + 8 * half])), acc);
+  if (li < a.H) {
+    const float off = sOff[32 * nb + li];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int pb = p0 + 8 * c + 4 * half;
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int pe = pb + e;
+        const int za = a.transpose ? pe : r, zb = a.transpose ? r : pe;
+        float b = (acc[4 * c + e] + off) * SF_LOG2E;
+        if (zb >= a.N) b = -INFINITY;
+        else if (za >= a.N) b = 0.f;
+        else if (((mbits >> (pe - p0)) & 1u) == 0) b = SF_MASKED_LOGIT;
+        v[e] = b;
+      }
+      if (!a.transpose) {   // za = r: four consecutive keys of one bias row (stored together)
+        *reinterpret_cast<u32x2*>(a.bias + bias_off(li, r, pb, a.NP)) = u32x2{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+      } else {              // zb = r: one key of four bias rows
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a.bias[bias_off(li, pb + e, r, a.NP)] = f2bf(v[e]);
+      }
+    }
+  }
+}
+
 // Persistent: each workgroup keeps the folded weight in LDS and walks 32-position blocks;
 // positions of attention row r are z[r, p] (starting node) or z[p, r] (ending node).
 // A block of 32 projection rows is one head of 32 dims (KC = 2) or two heads of 16 (KC = 1,
@@ -256,7 +363,7 @@ __global__ __launch_bounds__(64 * kPWaves) void tri_proj_kernel(const TriProjArg
   __shared__ __attribute__((aligned(16))) float sOff[PB * 32];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, li = lane & 31;
-  const int N = a.N, NP = a.NP, H = a.H;
+  const int N = a.N, NP = a.NP;
 
   // every load is issued before the first LDS store: one memory latency for the whole staging
   // (a loop of load, wait, store paid it 13 times per workgroup)
@@ -293,8 +400,6 @@ __global__ __launch_bounds__(64 * kPWaves) void tri_proj_kernel(const TriProjArg
 #pragma unroll
     for (int kk = 0; kk < NC; ++kk) x[kk] = ld16(zp + 16 * kk);
   };
-  auto pos_valid = [&](int r, int pe) { return a.transpose ? (pe < N && r < N) : (r < N && pe < N); };
-
   const int first = (blockIdx.x * kPWaves + wave) * a.items_per_wave;
   const int last = min(first + a.items_per_wave, a.items);
   if (first >= last) return;                            // uniform: no barrier follows
@@ -318,103 +423,15 @@ __global__ __launch_bounds__(64 * kPWaves) void tri_proj_kernel(const TriProjArg
     if (item + 2 < last) block_load(item + 2, fut.x, fut.v, fut.r, fut.p, fut.sm);
     const int p0 = p - li;
 
-    // q, k: D^T = W . X^T -> lane = position; registers 8*kk .. 8*kk+7 are the 16 bytes of
-    // k-chunk kk (KC = 2) or of head 2 nb + kk (KC = 1) in the Q/K layout
+    // (no branch around the stores: the compiler could not count them, and the waits for the next
+    // item's z would include them)
 #pragma unroll
-    for (int which = 0; which < 2; ++which) {
-      uint16_t* dst = which == 0 ? a.q : a.k;
-      const float sc = which == 0 ? a.qscale : 1.0f;
+    for (int which = 0; which < 2; ++which)
 #pragma unroll
-      for (int hh = 0; hh < NB; ++hh) {
-        const int nb = NB * which + hh;
-        f32x16 acc;
+      for (int hh = 0; hh < NB; ++hh) proj_qk_block<KC>(a, which, hh, sW, sOff, NB * which + hh, xo, valid, r, p, lane);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-#pragma unroll
-        for (int kk = 0; kk < NC; ++kk)
-          acc = mfma32(as_bf16x8(ld16(&sW[(32 * nb + li) * WP + 16 * kk + 8 * half])), xo[kk], acc);
-        // KC = 2: k-chunk kk of head hh, 512 elements apart; KC = 1: head 2 hh + kk (NP * 16 apart)
-        uint16_t* op = dst + ql_off<KC>(r, KC == 2 ? hh : 2 * hh, H, NP, p, 0, half);
-        constexpr int kStep = KC == 2 ? 512 : 0;
-        const int64_t step = KC == 2 ? kStep : (int64_t)NP * 16;
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-          const f32x4 o0 = *reinterpret_cast<const f32x4*>(&sOff[32 * nb + 16 * kk + 4 * half]);
-          const f32x4 o1 = *reinterpret_cast<const f32x4*>(&sOff[32 * nb + 16 * kk + 8 + 4 * half]);
-          uint32_t w[4];
-#pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            w[e] = pack_bf2(valid ? (acc[8 * kk + 2 * e] + o0[2 * e]) * sc : 0.f,
-                            valid ? (acc[8 * kk + 2 * e + 1] + o0[2 * e + 1]) * sc : 0.f);
-            w[2 + e] = pack_bf2(valid ? (acc[8 * kk + 4 + 2 * e] + o1[2 * e]) * sc : 0.f,
-                                valid ? (acc[8 * kk + 4 + 2 * e + 1] + o1[2 * e + 1]) * sc : 0.f);
-          }
-          st16_stream(op + kk * step, u32x4{w[0], w[1], w[2], w[3]});
-        }
-      }
-    }
-    // v: D = X . W^T -> lane = projection row li (head hh, dim li for KC = 2; head 2 hh + li / 16,
-    // dim li % 16 for KC = 1); registers 8*cc .. 8*cc+7 are keys of 16-key chunk cc of this block
-    // in PV slot order for lane half `half`
-#pragma unroll
-    for (int hh = 0; hh < NB; ++hh) {
-      const int nb = 2 * NB + hh;
-      f32x16 acc;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-#pragma unroll
-      for (int kk = 0; kk < NC; ++kk)
-        acc = mfma32(xo[kk], as_bf16x8(ld16(&sW[(32 * nb + li) * WP + 16 * kk + 8 * half])), acc);
-      const float off = sOff[32 * nb + li];
-      const int vh = KC == 2 ? hh : 2 * hh + (li >> 4), vd = KC == 2 ? li : li & 15;
-#pragma unroll
-      for (int cc = 0; cc < 2; ++cc) {
-        uint32_t w[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int t0 = 2 * e, t1 = 2 * e + 1;         // slot t -> key 16cc + 8(t/4) + 4half + t%4
-          const int k0 = p0 + 16 * cc + 8 * (t0 >> 2) + 4 * half + (t0 & 3);
-          const int k1 = p0 + 16 * cc + 8 * (t1 >> 2) + 4 * half + (t1 & 3);
-          w[e] = pack_bf2(pos_valid(r, k0) ? acc[8 * cc + t0] + off : 0.f,
-                          pos_valid(r, k1) ? acc[8 * cc + t1] + off : 0.f);
-        }
-        st16_stream(a.vt + vl_off<KC>(r, vh, H, NP, (p0 >> 4) + cc, half, vd), u32x4{w[0], w[1], w[2], w[3]});
-      }
-    }
-    // bias planes: D = X . Wb^T, lane = head li (< H), 4 consecutive positions
-    {
-      const int nb = 3 * NB;                            // LDS block of the folded bias rows
-      f32x16 acc;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-#pragma unroll
-      for (int kk = 0; kk < NC; ++kk)
-        acc = mfma32(xo[kk], as_bf16x8(ld16(&sW[(32 * nb + li) * WP + 16 * kk + 8 * half])), acc);
-      if (li < H) {
-        const float off = sOff[32 * nb + li];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const int pb = p0 + 8 * c + 4 * half;
-          float v[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int pe = pb + e;
-            const int za = a.transpose ? pe : r, zb = a.transpose ? r : pe;
-            float b = (acc[4 * c + e] + off) * SF_LOG2E;
-            if (zb >= N) b = -INFINITY;
-            else if (za >= N) b = 0.f;
-            else if (((mbits >> (pe - p0)) & 1u) == 0) b = SF_MASKED_LOGIT;
-            v[e] = b;
-          }
-          if (!a.transpose) {   // za = r: four consecutive keys of one bias row (stored together)
-            *reinterpret_cast<u32x2*>(a.bias + bias_off(li, r, pb, NP)) = u32x2{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
-          } else {              // zb = r: one key of four bias rows
-#pragma unroll
-            for (int e = 0; e < 4; ++e) a.bias[bias_off(li, pb + e, r, NP)] = f2bf(v[e]);
-          }
-        }
-      }
-    }
+    for (int hh = 0; hh < NB; ++hh) proj_v_block<KC>(a, hh, sW, sOff, 2 * NB + hh, xo, r, p0, lane);
+    proj_bias_block<KC>(a, sW, sOff, 3 * NB, xo, mbits, r, p0, lane);
     if (item + 1 < last) {
       ln_operands<NC>(nxt.x, nxt.v, xo);
       int smn = nxt.sm;
@@ -426,6 +443,49 @@ __global__ __launch_bounds__(64 * kPWaves) void tri_proj_kernel(const TriProjArg
   for (int item = first; item < last; item += 2) {
     iteration(item, zb_, za_);
     if (item + 1 < last) iteration(item + 1, za_, zb_);
+  }
+}
+
+// The same for few positions: a block of 32 folded rows per workgroup (blockIdx.y) and an item per
+// wave, so that a small pair representation spreads over the chip.  One wave of the kernel above
+// takes an item through all PB blocks in turn, and every workgroup first stages all of W: 14 us
+// whatever N, of which staging took 1.6, LayerNorm 0.9 and the blocks 9 (N = 20).
+constexpr int kSplitWaves = 4;
+
+template <int KC>
+__global__ __launch_bounds__(64 * kSplitWaves) void tri_proj_split_kernel(const TriProjArgs a) {
+  using TD = TriDims<KC>;
+  constexpr int C = TD::C, WP = TD::WP, NC = TD::NC, NB = TD::NB;
+  __shared__ __attribute__((aligned(16))) uint16_t sW[32 * WP];
+  __shared__ __attribute__((aligned(16))) float sOff[32];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5, li = lane & 31;
+  const int N = a.N, nb = blockIdx.y;                   // 0 .. 3 NB - 1: q, k, v; 3 NB: bias
+  const int bpr = a.NP / 32, item = blockIdx.x * kSplitWaves + wave;   // (a.items is a multiple of kSplitWaves)
+  const int r = item / bpr, p0 = (item - r * bpr) * 32, p = p0 + li;
+  const int za = a.transpose ? p : r, zb = a.transpose ? r : p;
+  const bool valid = za < N && zb < N;
+  const int sm = a.seq[valid ? zb : 0];
+  const uint16_t* zp = a.z + ((int64_t)(valid ? za : 0) * N + (valid ? zb : 0)) * C + 8 * half;
+  u32x4 x[NC];
+#pragma unroll
+  for (int kk = 0; kk < NC; ++kk) x[kk] = ld16(zp + 16 * kk);
+  const int src = nb < 3 * NB ? 32 * nb : 4 * C;        // first folded row of the block
+  constexpr int kStage = 32 * (C / 8) / (64 * kSplitWaves);
+#pragma unroll
+  for (int j = 0; j < kStage; ++j) {
+    const int t = tid + j * 64 * kSplitWaves, n = t / (C / 8), c8 = (t % (C / 8)) * 8;
+    st16(&sW[n * WP + c8], ld16(a.wf + (int64_t)(src + n) * C + c8));
+  }
+  if (tid < 32) sOff[tid] = a.off[src + tid];
+  bf16x8 xo[NC];
+  ln_operands<NC>(x, valid, xo);
+  __syncthreads();
+  if (nb == 3 * NB) {                                   // uniform, as below
+    proj_bias_block<KC>(a, sW, sOff, 0, xo, (uint32_t)__ballot(sm != 0), r, p0, lane);
+  } else if (r < N) {   // (the attention kernel computes row groups of 4 and stores rows below N only)
+    if (nb < 2 * NB) proj_qk_block<KC>(a, nb / NB, nb % NB, sW, sOff, 0, xo, valid, r, p, lane);
+    else proj_v_block<KC>(a, nb - 2 * NB, sW, sOff, 0, xo, r, p0, lane);
   }
 }
 
@@ -482,6 +542,47 @@ __device__ __forceinline__ void stage_out_weights(uint16_t* sW, uint16_t* sG, fl
   for (int n = tid; n < C; n += NTHR) sGoff[n] = goff[n];
 }
 
+// Gate block nb of 32 positions applied to the two o pieces of its chunks 2nb and 2nb + 1: D^T = W_g . X^T -> lane (position, half hf) holds gate row 8c + 4hf + e of the
+// block in register 4c + e.
+//  KC = 2 (block = head nb): o operand chunk kk = 2nb + j of lane half h needs the gate of
+//    half j, register 8h + t -- one permlane32 swap per register pair gets it.
+//  KC = 1 (block = heads 2nb, 2nb + 1): chunk kk = 2nb + j of lane half h needs dims
+//    8(t/4) + 4h + t%4 of head 2nb + j: rows 16j + ..., register 8j + t of the same lane half.
+template <int KC>
+__device__ __forceinline__ void gate_block(const u32x4* on, const bf16x8 (&zo)[TriDims<KC>::NC], const uint16_t* sG,
+                                           const float* sGoff, int nb, int lane, bf16x8* xg) {
+  constexpr int NC = TriDims<KC>::NC, WP = TriDims<KC>::WP;
+  const int half = lane >> 5, li = lane & 31;
+  f32x16 acc;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+#pragma unroll
+  for (int kk = 0; kk < NC; ++kk)
+    acc = mfma32(as_bf16x8(ld16(&sG[(32 * nb + li) * WP + 16 * kk + 8 * half])), zo[kk], acc);
+  float sg[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) sg[r] = sigmoidf_(acc[r] + sGoff[32 * nb + 8 * (r >> 2) + 4 * half + (r & 3)]);
+  if constexpr (KC == 2) {
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(sg[t]), __float_as_uint(sg[t + 8]), false, false);
+      // sw[0]: gate for chunk 2nb (j = 0), sw[1]: for chunk 2nb + 1 (j = 1), element t
+      sg[t] = __uint_as_float(sw[0]);
+      sg[t + 8] = __uint_as_float(sw[1]);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const u32x4 w = on[j];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const bf16x2 v = cvt_bf2(bflo(w[e]) * sg[8 * j + 2 * e], bfhi(w[e]) * sg[8 * j + 2 * e + 1]);
+      xg[j][2 * e] = v[0];
+      xg[j][2 * e + 1] = v[1];
+    }
+  }
+}
+
 // Gate of 32 pair positions (lane = position li, half = channel half): from this lane's z
 // channels 16 kk + 8 half + 0..7 (zn) and o pieces (on: feature 16 kk + 8 half + 0..7 of o is,
 // for KC = 2, head kk/2, piece (hf = kk%2, k-chunk = half) of the epilogue's order; for KC = 1,
@@ -494,8 +595,7 @@ template <int KC = 2>
 __device__ __forceinline__ void out_gate(const u32x4 (&on)[TriDims<KC>::NC], const u32x4 (&zn)[TriDims<KC>::NC], bool ok,
                                          bool add_residual, const uint16_t* sG, const float* sGoff, int lane,
                                          bf16x8 (&xg)[TriDims<KC>::NC], uint32_t (&zr)[TriDims<KC>::NC][2][2]) {
-  constexpr int NC = TriDims<KC>::NC, NB = TriDims<KC>::NB, WP = TriDims<KC>::WP;
-  const int half = lane >> 5, li = lane & 31;
+  constexpr int NC = TriDims<KC>::NC, NB = TriDims<KC>::NB;
   bf16x8 zo[NC];
   ln_operands<NC>(zn, ok, zo);
   if (add_residual) {   // (add_residual false: the caller supplies the residual another way, or none)
@@ -510,43 +610,8 @@ __device__ __forceinline__ void out_gate(const u32x4 (&on)[TriDims<KC>::NC], con
       }
     }
   }
-  // gate block nb: D^T = W_g . X^T -> lane (position, half hf) holds gate row 8c + 4hf + e of the
-  // block in register 4c + e.
-  //  KC = 2 (block = head nb): o operand chunk kk = 2nb + j of lane half h needs the gate of
-  //    half j, register 8h + t -- one permlane32 swap per register pair gets it.
-  //  KC = 1 (block = heads 2nb, 2nb + 1): chunk kk = 2nb + j of lane half h needs dims
-  //    8(t/4) + 4h + t%4 of head 2nb + j: rows 16j + ..., register 8j + t of the same lane half.
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb) {
-    f32x16 acc;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-#pragma unroll
-    for (int kk = 0; kk < NC; ++kk)
-      acc = mfma32(as_bf16x8(ld16(&sG[(32 * nb + li) * WP + 16 * kk + 8 * half])), zo[kk], acc);
-    float sg[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) sg[r] = sigmoidf_(acc[r] + sGoff[32 * nb + 8 * (r >> 2) + 4 * half + (r & 3)]);
-    if constexpr (KC == 2) {
-#pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(sg[t]), __float_as_uint(sg[t + 8]), false, false);
-        // sw[0]: gate for chunk 2nb (j = 0), sw[1]: for chunk 2nb + 1 (j = 1), element t
-        sg[t] = __uint_as_float(sw[0]);
-        sg[t + 8] = __uint_as_float(sw[1]);
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const u32x4 w = on[2 * nb + j];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const bf16x2 v = cvt_bf2(bflo(w[e]) * sg[8 * j + 2 * e], bfhi(w[e]) * sg[8 * j + 2 * e + 1]);
-        xg[2 * nb + j][2 * e] = v[0];
-        xg[2 * nb + j][2 * e + 1] = v[1];
-      }
-    }
-  }
+  for (int nb = 0; nb < NB; ++nb) gate_block<KC>(&on[2 * nb], zo, sG, sGoff, nb, lane, &xg[2 * nb]);
 }
 
 // Output projection + residual of the 32 positions: out[p] = z[p] + (o[p] * g[p]) . W_o^T
@@ -658,6 +723,73 @@ __global__ __launch_bounds__(64 * kPWaves) void tri_out_kernel(const TriOutArgs 
       out_gate<KC>(on, zn, inn < a.N, a.add_residual, sG, sGoff, lane, xg, zr);
       r = rn; in = inn;
     }
+  }
+}
+
+// The same for few positions: an item per workgroup, a gate and an output block per wave.  Wave w
+// normalises z itself, forms gate block w and puts its two chunks of gated o into LDS; then every
+// wave forms its 32 output channels from all of them.  (An item per wave took 10 us whatever N.)
+// After the gate, the rows of W_g hold the waves' output rows.
+template <int KC>
+__global__ __launch_bounds__(64 * TriDims<KC>::NB) void tri_out_split_kernel(const TriOutArgs a) {
+  using TD = TriDims<KC>;
+  constexpr int C = TD::C, WP = TD::WP, NC = TD::NC, NB = TD::NB;
+  constexpr int kOP = 36;                               // pitch (elements) of a wave's 32 x 32 output rows
+  static_assert(NB * 32 * kOP <= C * WP, "the output rows fit where W_g was");
+  __shared__ __attribute__((aligned(16))) uint16_t sW[C * WP];
+  __shared__ __attribute__((aligned(16))) uint16_t sG[C * WP];
+  __shared__ __attribute__((aligned(16))) float sGoff[C];
+  __shared__ __attribute__((aligned(16))) uint16_t sX[NC * 64 * 8];   // gated o operands, 16 bytes a lane
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5, li = lane & 31;
+  const int IB = (a.N + 31) >> 5, r = blockIdx.x / IB, i0 = (blockIdx.x - r * IB) * 32;
+  auto pos = [&](int i) -> int64_t { return a.transpose ? (int64_t)i * a.N + r : (int64_t)r * a.N + i; };
+  const bool ok = i0 + li < a.N;
+  const int i = ok ? i0 + li : 0;                       // lanes past N: query 0, never stored
+  const uint16_t* zp = a.z + pos(i) * C;
+  u32x4 zn[NC], on[2];
+  u32x2 zr[4];                                          // residual: this lane's output channels
+#pragma unroll
+  for (int kk = 0; kk < NC; ++kk) zn[kk] = ld16(zp + 16 * kk + 8 * half);
+#pragma unroll
+  for (int j = 0; j < 2; ++j) on[j] = ld16(a.o + o_piece_off<KC>(2 * wave + j, r, i, half, a.N, a.NP));
+#pragma unroll
+  for (int c = 0; c < 4; ++c) zr[c] = *reinterpret_cast<const u32x2*>(zp + 32 * wave + 8 * c + 4 * half);
+  stage_out_weights<64 * NB, KC>(sW, sG, sGoff, a.wo, a.wg, a.goff, tid);
+  bf16x8 zo[NC], xg[NC];
+  ln_operands<NC>(zn, ok, zo);
+  __syncthreads();
+  bf16x8 own[2];
+  gate_block<KC>(on, zo, sG, sGoff, wave, lane, own);
+#pragma unroll
+  for (int j = 0; j < 2; ++j) *reinterpret_cast<bf16x8*>(&sX[((2 * wave + j) * 64 + lane) * 8]) = own[j];
+  __syncthreads();
+#pragma unroll
+  for (int kk = 0; kk < NC; ++kk) xg[kk] = as_bf16x8(ld16(&sX[(kk * 64 + lane) * 8]));
+  f32x16 acc;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+#pragma unroll
+  for (int kk = 0; kk < NC; ++kk)
+    acc = mfma32(as_bf16x8(ld16(&sW[(32 * wave + li) * WP + 16 * kk + 8 * half])), xg[kk], acc);
+  uint16_t* const so = sG + wave * 32 * kOP;            // (no wave reads W_g past the barrier above)
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = acc[4 * c + e];
+    if (a.add_residual) {
+      v[0] += bflo(zr[c][0]); v[1] += bfhi(zr[c][0]); v[2] += bflo(zr[c][1]); v[3] += bfhi(zr[c][1]);
+    }
+    *reinterpret_cast<u32x2*>(so + li * kOP + 8 * c + 4 * half) = u32x2{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+  }
+  asm volatile("" ::: "memory");                        // one wave's LDS accesses run in order
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {                         // 16 rows of 64 bytes per store
+    const int row = 16 * u + (lane >> 2), ch = (lane & 3) * 8;
+    const u32x2 lo = *reinterpret_cast<const u32x2*>(so + row * kOP + ch);
+    const u32x2 hi = *reinterpret_cast<const u32x2*>(so + row * kOP + ch + 4);
+    if (i0 + row < a.N) st16(a.out + pos(i0 + row) * C + 32 * wave + ch, u32x4{lo[0], lo[1], hi[0], hi[1]});
   }
 }
 
@@ -1959,6 +2091,13 @@ float sum_limit(float requested) {
   return requested > 0.f && requested <= v ? requested : v;
 }
 
+// Items (of 32 positions) up to which the projection and the output stage run split: two waves per
+// SIMD of the unsplit kernels' 8-wave workgroups would then fill at most a quarter of the chip.
+// Whole call at C = 128, us, unsplit against split (the host takes 35 of it): projection N = 64
+// 37.7 / 35.9, 150 (2048 items) 47.5 / 59.4; output N = 64 37.7 / 34.2, 128 (512) 39.1 / 37.5,
+// 150 (750) 47.5 / 49.3, 200 (1400) 50.1 / 60.3.
+constexpr int kSplitItems = 512;
+
 template <int KC>
 int triangle_fast(const sf_triangle_args* a, void* workspace, size_t workspace_bytes, hipStream_t st, int stages) {
   using TD = TriDims<KC>;
@@ -1988,8 +2127,12 @@ int triangle_fast(const sf_triangle_args* a, void* workspace, size_t workspace_b
     pa.wf = ws.wf; pa.off = ws.off;
     pa.q = ws.q; pa.k = ws.k; pa.vt = ws.vt; pa.bias = ws.bias;
     pa.items = NP * (NP / 32);
-    const int pgroups = persistent_groups(pa.items, &pa.items_per_wave);
-    hipLaunchKernelGGL(tri_proj_kernel<KC>, dim3(pgroups), dim3(64 * kPWaves), 0, st, pa);
+    if (pa.items <= kSplitItems) {
+      hipLaunchKernelGGL(tri_proj_split_kernel<KC>, dim3(pa.items / kSplitWaves, TD::ProjBlocks), dim3(64 * kSplitWaves), 0, st, pa);
+    } else {
+      const int pgroups = persistent_groups(pa.items, &pa.items_per_wave);
+      hipLaunchKernelGGL(tri_proj_kernel<KC>, dim3(pgroups), dim3(64 * kPWaves), 0, st, pa);
+    }
     if (int rc = sf_check_launch("tri_proj_kernel")) return rc;
   }
 
@@ -2031,8 +2174,12 @@ int triangle_fast(const sf_triangle_args* a, void* workspace, size_t workspace_b
   oa.z = (const uint16_t*)a->z; oa.add_residual = a->add_residual;
   oa.out = (uint16_t*)a->out;
   oa.items = N * ((N + 31) / 32);
-  const int ogroups = persistent_groups(oa.items, &oa.items_per_wave);
-  hipLaunchKernelGGL(tri_out_kernel<KC>, dim3(ogroups), dim3(64 * kPWaves), 0, st, oa);
+  if (oa.items <= kSplitItems) {
+    hipLaunchKernelGGL(tri_out_split_kernel<KC>, dim3(oa.items), dim3(64 * TD::NB), 0, st, oa);
+  } else {
+    const int ogroups = persistent_groups(oa.items, &oa.items_per_wave);
+    hipLaunchKernelGGL(tri_out_kernel<KC>, dim3(ogroups), dim3(64 * kPWaves), 0, st, oa);
+  }
   return sf_check_launch("tri_out_kernel");
 }
 }  // namespace

@@ -78,9 +78,47 @@ struct ProjArgs {
   int items, items_per_wave;     // blocks of 32 plane columns: Pn rows x Pn / 32
 };
 
-// D^T = W X^T per 32 channels x 32 positions: lane (li, half) ends with position li (plane column
-// 32 cb + li) at channels 32 nb + 8(r/4) + 4 half + r%4; each register is one 2-byte store, and
-// the 32 lanes of a half write 64 contiguous bytes of one plane row.
+// item -> plane row R, columns 32 cb .. 32 cb + 31; this lane's column col.  Outgoing: z position
+// (R, col); incoming: (col, R), so that the planes hold a^T and b^T
+__device__ __forceinline__ void load_item(const ProjArgs& a, int item, int li, int half, u32x4 (&zn)[8], bool& ok, int& R, int& col,
+                                          int& m0, int& m1) {
+  const int cbs = a.Pn / 32;                            // column blocks per plane row
+  R = item / cbs;
+  col = 32 * (item - R * cbs) + li;
+  const int za = a.incoming ? col : R, zb = a.incoming ? R : col;
+  ok = za < a.N && zb < a.N;
+  const uint16_t* zp = a.z + (ok ? (int64_t)za * a.N + zb : 0) * kC + 8 * half;
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk) zn[kk] = ld16(zp + 16 * kk);
+  m0 = a.mask == nullptr ? 1 : a.mask[ok ? za : 0];
+  m1 = a.mask == nullptr ? 1 : a.mask[ok ? zb : 0];
+}
+
+// One block of 32 channels: gate rows wg and projection rows wp (LDS, pitch kWS), their offsets og
+// and op; plane of the block's first channel at dst, this lane's position at byte offset lofs.
+// D^T = W X^T: lane (li, half) ends with position li at channels 8(r/4) + 4 half + r%4 of the block;
+// each register is one 2-byte store, and the 32 lanes of a half write 64 contiguous bytes of one
+// plane row.
+__device__ __forceinline__ void proj_block(const uint16_t* wg, const uint16_t* wp, const float* og, const float* op,
+                                           const bf16x8 (&xo)[8], bool keep, char* dst, int64_t pstride, int64_t lofs, int lane) {
+  const int half = lane >> 5, li = lane & 31;
+  f32x16 ag, ap;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) { ag[e] = 0.f; ap[e] = 0.f; }
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk) {
+    ag = mfma32(as_bf16x8(ld16(&wg[li * kWS + 16 * kk + 8 * half])), xo[kk], ag);
+    ap = mfma32(as_bf16x8(ld16(&wp[li * kWS + 16 * kk + 8 * half])), xo[kk], ap);
+  }
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int ch = 8 * (r >> 2) + 4 * half + (r & 3);               // this register's channel
+    const float v = sigmoidf_(ag[r] + og[ch]) * (ap[r] + op[ch]);
+    char* cbase = dst + (int64_t)(8 * (r >> 2) + (r & 3)) * pstride * 2;   // uniform
+    *reinterpret_cast<uint16_t*>(cbase + lofs) = f2bf(keep ? v : 0.f);
+  }
+}
+
 // No wait covers a store: the next item's z rows and mask bytes are loaded before this item's
 // products, unconditionally (positions past N read position 0; their values are replaced by
 // zeros), and normalised after its stores.  With the loads predicated, the mask read between the
@@ -105,31 +143,17 @@ __global__ __launch_bounds__(64 * kTW) void trimul_proj_kernel(const ProjArgs a)
   }
   for (int n = tid; n < kGlu; n += 64 * kTW) sOff[n] = a.off[n];
   __syncthreads();
-  const int cbs = a.Pn / 32;                            // column blocks per plane row
   const int64_t plane = (int64_t)a.Pn * a.Pn;
   // the workgroup's items are base .. base + kTW * items_per_wave - 1, wave w taking every kTW-th:
   // neighbouring column blocks, whose stores fill the two halves of each 128-byte plane line, are
   // written together (one wave walking consecutive items came back to a line too late for L2)
   const int base = blockIdx.x * kTW * a.items_per_wave;
-  // item -> plane row R, columns 32 cb .. 32 cb + 31; this lane's column col.  Outgoing: z position
-  // (R, col); incoming: (col, R), so that the planes hold a^T and b^T
-  auto load_item = [&](int item, u32x4 (&zn)[8], bool& ok, int& R, int& col, int& m0, int& m1) __attribute__((always_inline)) {
-    R = item / cbs;
-    col = 32 * (item - R * cbs) + li;
-    const int za = a.incoming ? col : R, zb = a.incoming ? R : col;
-    ok = za < a.N && zb < a.N;
-    const uint16_t* zp = a.z + (ok ? (int64_t)za * a.N + zb : 0) * kC + 8 * half;
-#pragma unroll
-    for (int kk = 0; kk < 8; ++kk) zn[kk] = ld16(zp + 16 * kk);
-    m0 = a.mask == nullptr ? 1 : a.mask[ok ? za : 0];
-    m1 = a.mask == nullptr ? 1 : a.mask[ok ? zb : 0];
-  };
   int item = base + wave;
   if (item >= a.items) return;                        // uniform: no barrier follows
   u32x4 zn[8];
   bool ok;
   int R, col, m0, m1;
-  load_item(item, zn, ok, R, col, m0, m1);
+  load_item(a, item, li, half, zn, ok, R, col, m0, m1);
   bf16x8 xo[8];
   ln128_operands(zn, ok, xo);
   bool keep = ok && m0 != 0 && m1 != 0;
@@ -139,7 +163,7 @@ __global__ __launch_bounds__(64 * kTW) void trimul_proj_kernel(const ProjArgs a)
     const bool more = k + 1 < a.items_per_wave && nitem < a.items;   // uniform
     bool okn = false;
     int Rn = 0, coln = 0, m0n = 0, m1n = 0;
-    if (more) load_item(nitem, zn, okn, Rn, coln, m0n, m1n);
+    if (more) load_item(a, nitem, li, half, zn, okn, Rn, coln, m0n, m1n);
     // store address = a uniform base per channel (scalar registers, recomputed every item from an
     // opaque plane stride; hoisted, the 16 channel offsets of each block took 32 VGPRs) plus this
     // lane's byte offset (half 4 planes in, plus the position; 64-bit: four planes pass 4 GiB
@@ -152,23 +176,9 @@ __global__ __launch_bounds__(64 * kTW) void trimul_proj_kernel(const ProjArgs a)
       char* dstp = reinterpret_cast<char*>(side ? a.b : a.a);
 #pragma unroll
       for (int nb = 0; nb < kC / 32; ++nb) {
-        const int rg = side * kC + 32 * nb + li;        // gate row of this lane's channel
-        const int rp = 2 * kC + rg;                     // projection row
-        f32x16 ag, ap;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) { ag[e] = 0.f; ap[e] = 0.f; }
-#pragma unroll
-        for (int kk = 0; kk < 8; ++kk) {
-          ag = mfma32(as_bf16x8(ld16(&sW[rg * kWS + 16 * kk + 8 * half])), xo[kk], ag);
-          ap = mfma32(as_bf16x8(ld16(&sW[rp * kWS + 16 * kk + 8 * half])), xo[kk], ap);
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int ch = 32 * nb + 8 * (r >> 2) + 4 * half + (r & 3);   // this register's channel
-          const float v = sigmoidf_(ag[r] + sOff[side * kC + ch]) * (ap[r] + sOff[2 * kC + side * kC + ch]);
-          char* cbase = dstp + (int64_t)(32 * nb + 8 * (r >> 2) + (r & 3)) * pstride * 2;   // uniform
-          *reinterpret_cast<uint16_t*>(cbase + lofs) = f2bf(keep ? v : 0.f);
-        }
+        const int rg = side * kC + 32 * nb;             // first gate row of the block
+        proj_block(&sW[rg * kWS], &sW[(2 * kC + rg) * kWS], sOff + rg, sOff + 2 * kC + rg, xo, keep,
+                   dstp + (int64_t)32 * nb * pstride * 2, pstride, lofs, lane);
       }
     }
     if (!more) break;
@@ -177,6 +187,38 @@ __global__ __launch_bounds__(64 * kTW) void trimul_proj_kernel(const ProjArgs a)
     keep = okn && m0n != 0 && m1n != 0;
     item = nitem; R = Rn; col = coln;
   }
+}
+
+// The same for few positions: a block of 32 channels of one side per workgroup (blockIdx.y) and an
+// item per wave, so that a small pair representation spreads over the chip.  One wave of the kernel
+// above takes an item through all 8 blocks in turn, and every workgroup first stages all of W: 15 us
+// whatever N, of which staging took 1.6, LayerNorm 0.9 and the blocks 9 (N = 20).
+constexpr int kSplitWaves = 4;
+
+__global__ __launch_bounds__(64 * kSplitWaves) void trimul_proj_split_kernel(const ProjArgs a) {
+  __shared__ __attribute__((aligned(16))) uint16_t sW[64 * kWS];     // 32 gate rows, 32 projection rows
+  __shared__ float sOff[64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5, li = lane & 31;
+  const int rg = 32 * blockIdx.y;                                    // first gate row: side kC + 32 nb
+  const int item = blockIdx.x * kSplitWaves + wave;                  // (a.items is a multiple of kSplitWaves)
+  u32x4 zn[8];
+  bool ok;
+  int R, col, m0, m1;
+  load_item(a, item, li, half, zn, ok, R, col, m0, m1);
+#pragma unroll
+  for (int j = 0; j < 64 * (kC / 8) / (64 * kSplitWaves); ++j) {
+    const int t = tid + j * 64 * kSplitWaves, n = t >> 4, c8 = (t & 15) * 8;
+    st16(&sW[n * kWS + c8], ld16(a.w + (int64_t)((n >> 5) * 2 * kC + rg + (n & 31)) * kC + c8));
+  }
+  if (tid < 64) sOff[tid] = a.off[(tid >> 5) * 2 * kC + rg + (tid & 31)];
+  bf16x8 xo[8];
+  ln128_operands(zn, ok, xo);
+  __syncthreads();
+  const int64_t pstride = (int64_t)a.Pn * a.Pn;
+  char* dstp = reinterpret_cast<char*>(rg >= kC ? a.b : a.a) + (int64_t)(rg & (kC - 1)) * pstride * 2;
+  proj_block(sW, sW + 32 * kWS, sOff, sOff + 32, xo, ok && m0 != 0 && m1 != 0, dstp, pstride,
+             (4 * half * pstride + (int64_t)R * a.Pn + col) * 2, lane);
 }
 
 struct OutArgs {
@@ -192,6 +234,15 @@ struct OutArgs {
   uint16_t* out;                 // [P, 128]
   int items, items_per_wave;     // blocks of 32 of the P positions
 };
+
+// Position p of the product plane (below 2^31: N <= 8192) as one of z and out: the same where rows
+// are unpadded (N a multiple of 8); -1 past the end and at a padding column
+__device__ __forceinline__ int out_position(const OutArgs& a, int p) {
+  if (p >= a.P) return -1;
+  if (a.Nt == a.N) return p;
+  const int row = p / a.Nt, col = p - row * a.Nt;
+  return col < a.N ? row * a.N + col : -1;
+}
 
 // D^T = W X^T per 32 output channels x 32 positions: lane (li, half) ends with position li at
 // channels 32 nb + 8(r/4) + 4 half + r%4; the gated update (plus the residual, taken from the z
@@ -228,14 +279,7 @@ __global__ __launch_bounds__(64 * kTW) void trimul_out_kernel(const OutArgs a) {
   for (int k = 0; k < a.items_per_wave; ++k) {
     const int item = base + k * kTW + wave;
     if (item >= a.items) break;
-    // this lane's position of the product plane (below 2^31: N <= 8192) as one of z and out: the
-    // same where rows are unpadded (N a multiple of 8); -1 past the end and at a padding column
-    int p = item * 32 + li;
-    if (p >= a.P) p = -1;
-    if (a.Nt != a.N && p >= 0) {
-      const int row = p / a.Nt, col = p - row * a.Nt;
-      p = col < a.N ? row * a.N + col : -1;
-    }
+    const int p = out_position(a, item * 32 + li);    // this lane's position, or -1
     // the block's product, [128 channels][32 positions] (64 contiguous bytes per channel): 16-byte
     // loads into the wave's LDS rows at pitch 34, then each lane reads channels 16 kk + 8 half + 0..7
     // of its position.  Positions past P read the plane's padding (Pp >= item * 32 + 32), unused.
@@ -324,6 +368,102 @@ __global__ __launch_bounds__(64 * kTW) void trimul_out_kernel(const OutArgs a) {
   }
 }
 
+// The same for few positions: an item per workgroup, a block of 32 output channels per wave.  (An
+// item per wave took 12.5 us whatever N: 1.3 of staging, 2 of loads, 1.4 of LayerNorm, 4 of blocks.)
+// The workgroup loads the block of t together, every wave normalises it and z for itself; the output
+// rows then take the place of t.
+__global__ __launch_bounds__(256) void trimul_out_split_kernel(const OutArgs a) {
+  constexpr int kOP = 36;                               // pitch (elements) of a wave's 32 x 32 output rows
+  __shared__ __attribute__((aligned(16))) uint16_t sWo[kC * kWS];
+  __shared__ __attribute__((aligned(16))) uint16_t sWg[kC * kWS];
+  __shared__ float sOo[kC], sOg[kC];
+  __shared__ __attribute__((aligned(16))) uint16_t sT[4 * 32 * kOP];
+  static_assert(4 * 32 * kOP >= kC * kTP, "t and the output rows share the space");
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5, li = lane & 31;
+  const int p = out_position(a, blockIdx.x * 32 + li);
+  u32x4 tv[2], zn[8];
+  u32x2 zr[4];                                          // residual: this lane's output channels
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int w = tid + 256 * u, c = w >> 2, seg = w & 3;
+    tv[u] = ld16(a.t + (int64_t)c * a.Pp + (int64_t)blockIdx.x * 32 + 8 * seg);
+  }
+  const uint16_t* zp = a.z + (int64_t)max(p, 0) * kC;
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk) zn[kk] = ld16(zp + 16 * kk + 8 * half);
+#pragma unroll
+  for (int g = 0; g < 4; ++g) zr[g] = *reinterpret_cast<const u32x2*>(zp + 32 * wave + 8 * g + 4 * half);
+  constexpr int kStage = kC * (kC / 8) / 256;
+  u32x4 so_[kStage], sg_[kStage];
+#pragma unroll
+  for (int u = 0; u < kStage; ++u) {
+    const int t = tid + u * 256;
+    so_[u] = ld16(a.wo + (int64_t)(t >> 4) * kC + (t & 15) * 8);
+    sg_[u] = ld16(a.wg + (int64_t)(t >> 4) * kC + (t & 15) * 8);
+  }
+  uint32_t* const tw = reinterpret_cast<uint32_t*>(sT);
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int w = tid + 256 * u, c = w >> 2, seg = w & 3;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tw[(c * kTP + 8 * seg) / 2 + e] = tv[u][e];
+  }
+  if (tid < kC) { sOo[tid] = a.oo[tid]; sOg[tid] = a.og[tid]; }
+#pragma unroll
+  for (int u = 0; u < kStage; ++u) {
+    const int t = tid + u * 256;
+    st16(&sWo[(t >> 4) * kWS + (t & 15) * 8], so_[u]);
+    st16(&sWg[(t >> 4) * kWS + (t & 15) * 8], sg_[u]);
+  }
+  bf16x8 to[8], zo[8];
+  ln128_operands(zn, p >= 0, zo);
+  __syncthreads();
+  u32x4 tn[8];
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t lo = sT[(16 * kk + 8 * half + 2 * e) * kTP + li];
+      const uint32_t hi = sT[(16 * kk + 8 * half + 2 * e + 1) * kTP + li];
+      tn[kk][e] = p >= 0 ? lo | (hi << 16) : 0u;
+    }
+  }
+  ln128_operands(tn, p >= 0, to);
+  __syncthreads();                                      // (t is overwritten below)
+  f32x16 ao, ag;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) { ao[e] = 0.f; ag[e] = 0.f; }
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk) {
+    ao = mfma32(as_bf16x8(ld16(&sWo[(32 * wave + li) * kWS + 16 * kk + 8 * half])), to[kk], ao);
+    ag = mfma32(as_bf16x8(ld16(&sWg[(32 * wave + li) * kWS + 16 * kk + 8 * half])), zo[kk], ag);
+  }
+  uint16_t* const so = sT + wave * 32 * kOP;
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int c0 = 32 * wave + 8 * g + 4 * half;
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = (ao[4 * g + e] + sOo[c0 + e]) * sigmoidf_(ag[4 * g + e] + sOg[c0 + e]);
+    uint32_t u0 = pack_bf2(v[0], v[1]), u1 = pack_bf2(v[2], v[3]);   // the bf16 update
+    if (a.add_residual) {                                            // out = update + z
+      u0 = pack_bf2(bflo(u0) + bflo(zr[g][0]), bfhi(u0) + bfhi(zr[g][0]));
+      u1 = pack_bf2(bflo(u1) + bflo(zr[g][1]), bfhi(u1) + bfhi(zr[g][1]));
+    }
+    *reinterpret_cast<u32x2*>(so + li * kOP + 8 * g + 4 * half) = u32x2{u0, u1};
+  }
+  asm volatile("" ::: "memory");                        // one wave's LDS accesses run in order
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {                         // 16 rows of 64 bytes per store
+    const int row = 16 * u + (lane >> 2), ch = (lane & 3) * 8;
+    const u32x2 lo = *reinterpret_cast<const u32x2*>(so + row * kOP + ch);
+    const u32x2 hi = *reinterpret_cast<const u32x2*>(so + row * kOP + ch + 4);
+    const int pp = __shfl(p, row);                      // lane row holds the block's position row
+    if (pp >= 0) st16(a.out + (int64_t)pp * kC + 32 * wave + ch, u32x4{lo[0], lo[1], hi[0], hi[1]});
+  }
+}
+
 struct Ws {
   uint16_t *wglu, *wout, *wgate;
   float *oglu, *oout, *ogate;
@@ -351,6 +491,13 @@ Ws carve(char* base, int N) {
 }
 
 size_t ws_bytes(int N) { return carve(nullptr, N).bytes; }
+
+// Items (of 32 positions) up to which the projection and the output stage run split: two waves per
+// SIMD of the unsplit kernels' 8-wave workgroups would then fill at most a quarter of the chip.
+// Whole call, us, unsplit against split: projection N = 64 36.4 / 27.7, 128 (512 items) 41.1 / 36.3,
+// 200 (2048) 52.2 / 62.1; output N = 64 36.4 / 30.6, 128 (512) 41.1 / 38.9, 150 (713) 49.0 / 49.0,
+// 200 (1250) 52.2 / 59.0.
+constexpr int kSplitItems = 512;
 
 int launch_grid(const void* kernel, int items) {
   const int waves = std::max(1, std::min(sf_resident_workgroups(kernel, 64 * kTW) * kTW, items));
@@ -412,10 +559,14 @@ extern "C" int sf_hip_triangle_mult_fwd(const sf_triangle_mult_args* a, void* wo
     pa.z = static_cast<const uint16_t*>(a->z); pa.mask = a->mask;
     pa.w = w.wglu; pa.off = w.oglu; pa.a = w.a; pa.b = w.b;
     pa.items = Pn * (Pn / 32);                          // every plane row, padding included
-    const int waves = launch_grid(reinterpret_cast<const void*>(trimul_proj_kernel), pa.items);
-    pa.items_per_wave = (pa.items + waves - 1) / waves;
-    const int groups = (pa.items + pa.items_per_wave * kTW - 1) / (pa.items_per_wave * kTW);
-    hipLaunchKernelGGL(trimul_proj_kernel, dim3(groups), dim3(64 * kTW), 0, st, pa);
+    if (pa.items <= kSplitItems) {
+      hipLaunchKernelGGL(trimul_proj_split_kernel, dim3(pa.items / kSplitWaves, 8), dim3(64 * kSplitWaves), 0, st, pa);
+    } else {
+      const int waves = launch_grid(reinterpret_cast<const void*>(trimul_proj_kernel), pa.items);
+      pa.items_per_wave = (pa.items + waves - 1) / waves;
+      const int groups = (pa.items + pa.items_per_wave * kTW - 1) / (pa.items_per_wave * kTW);
+      hipLaunchKernelGGL(trimul_proj_kernel, dim3(groups), dim3(64 * kTW), 0, st, pa);
+    }
     if ((rc = sf_check_launch("trimul_proj_kernel"))) return rc;
   }
 
@@ -437,9 +588,13 @@ extern "C" int sf_hip_triangle_mult_fwd(const sf_triangle_mult_args* a, void* wo
   oa.N = N; oa.Nt = Nt; oa.P = P; oa.Pp = Pp; oa.t = w.t; oa.z = static_cast<const uint16_t*>(a->z);
   oa.wo = w.wout; oa.oo = w.oout; oa.wg = w.wgate; oa.og = w.ogate;
   oa.add_residual = a->add_residual; oa.out = static_cast<uint16_t*>(a->out); oa.items = items;
-  const int waves = launch_grid(reinterpret_cast<const void*>(trimul_out_kernel), items);
-  oa.items_per_wave = (items + waves - 1) / waves;
-  const int groups = (items + oa.items_per_wave * kTW - 1) / (oa.items_per_wave * kTW);
-  hipLaunchKernelGGL(trimul_out_kernel, dim3(groups), dim3(64 * kTW), 0, st, oa);
+  if (items <= kSplitItems) {
+    hipLaunchKernelGGL(trimul_out_split_kernel, dim3(items), dim3(256), 0, st, oa);
+  } else {
+    const int waves = launch_grid(reinterpret_cast<const void*>(trimul_out_kernel), items);
+    oa.items_per_wave = (items + waves - 1) / waves;
+    const int groups = (items + oa.items_per_wave * kTW - 1) / (oa.items_per_wave * kTW);
+    hipLaunchKernelGGL(trimul_out_kernel, dim3(groups), dim3(64 * kTW), 0, st, oa);
+  }
   return sf_check_launch("trimul_out_kernel");
 }
