@@ -126,10 +126,13 @@ class GridSelfAttentionHipMixin:
   @graphs.graphed
   def _forward_dense(self, act: torch.Tensor, seq_mask: torch.Tensor, *, add_residual: bool) -> torch.Tensor:
     N = act.shape[-2]
+    b = self._buffers                     # (the module's attribute lookup would search three dicts for each)
+    ln_w, ln_b, w_qkvgb, w_o = b["_hip_ln_w"], b["_hip_ln_b"], b["_hip_w_qkvgb"], b["_hip_w_o"]
+    kw = {"num_head": self.config.num_head, "transpose": self.transpose, "add_residual": add_residual}
+    if act.ndim == 3:                                   # one pair block: no batch views around the call
+      return ops.triangle_attention(act, seq_mask, ln_w, ln_b, w_qkvgb, w_o, **kw).to(act.dtype)
     flat = act.reshape(-1, N, N, act.shape[-1])
-    outs = [ops.triangle_attention(z, seq_mask, self._hip_ln_w, self._hip_ln_b, self._hip_w_qkvgb, self._hip_w_o,
-                                   num_head=self.config.num_head, transpose=self.transpose,
-                                   add_residual=add_residual) for z in flat]
+    outs = [ops.triangle_attention(z, seq_mask, ln_w, ln_b, w_qkvgb, w_o, **kw) for z in flat]
     out = outs[0].unsqueeze(0) if len(outs) == 1 else torch.stack(outs)
     return out.reshape(act.shape).to(act.dtype)
 
@@ -435,7 +438,8 @@ class TransitionBlockHipMixin:
   @_require_native_preparation
   @graphs.graphed
   def forward(self, act: torch.Tensor, *, broadcast_dim: int | None = 0, add_residual: bool = True) -> torch.Tensor:
-    w = {"ln_w": self._hip_ln_w, "ln_b": self._hip_ln_b, "w1": self._hip_w1, "w2": self._hip_w2}
+    b = self._buffers
+    w = {"ln_w": b["_hip_ln_w"], "ln_b": b["_hip_ln_b"], "w1": b["_hip_w1"], "w2": b["_hip_w2"]}
     rows = act.reshape(-1, act.shape[-1])
     out = ops.transition_module(rows, None, w, add_residual=add_residual)
     return out.view(act.shape).to(act.dtype)
@@ -749,7 +753,8 @@ class TriangleMultiplicationHipMixin:
   @_require_native_preparation
   @graphs.graphed
   def forward(self, act: torch.Tensor, mask: torch.Tensor, *, add_residual: bool = True) -> torch.Tensor:
-    w = {k: getattr(self, "_hip_" + k) for k in ("ln_w", "ln_b", "w_glu", "cn_w", "cn_b", "w_out", "w_gate")}
+    b = self._buffers
+    w = {k: b["_hip_" + k] for k in ("ln_w", "ln_b", "w_glu", "cn_w", "cn_b", "w_out", "w_gate")}
     out = ops.triangle_multiplication(act, mask, w, incoming=self.equation in self.INCOMING_EQUATIONS,
                                       add_residual=add_residual)
     return out.to(act.dtype)

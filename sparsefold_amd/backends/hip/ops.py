@@ -18,8 +18,11 @@ from sparsefold_amd import _lib
 BF16 = torch.bfloat16
 
 
+# The small calls are bound by this file: a call of 20 residues spends longer here than its kernels
+# run.  Pointers and streams are passed as plain ints (every struct field and argument that takes one
+# is declared c_void_p), the device check reads ints, and messages are formatted only when raised.
 def _vp(t: torch.Tensor | None):
-  return None if t is None else C.c_void_p(t.data_ptr())
+  return None if t is None else t.data_ptr()
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
@@ -29,24 +32,24 @@ def _stream(t: torch.Tensor):
   """torch's current stream on t's device (the raw handle; the public accessor builds a Stream
   object per call, which costs more than some of the kernels it launches)."""
   if _raw_stream is not None:
-    return C.c_void_p(_raw_stream(t.device.index))
-  return C.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return _raw_stream(t.get_device())
+  return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def _require_cuda(*ts: torch.Tensor | None) -> torch.device:
-  dev = None
+  first, index = None, -1
   for t in ts:
     if t is None:
       continue
-    if t.device.type != "cuda":
+    if not t.is_cuda:
       raise ValueError(f"HIP kernels need device tensors, got a tensor on {t.device}")
-    if dev is None:
-      dev = t.device
-    elif t.device != dev:
-      raise ValueError(f"tensors on different devices: {dev} and {t.device}")
-  if dev is None:
+    if first is None:
+      first, index = t, t.get_device()
+    elif t.get_device() != index:
+      raise ValueError(f"tensors on different devices: {first.device} and {t.device}")
+  if first is None:
     raise ValueError("no device tensor given")
-  return dev
+  return first.device
 
 
 def _require(cond: bool, msg: str) -> None:
@@ -258,13 +261,16 @@ def triangle_attention(z: torch.Tensor, seq_mask: torch.Tensor, ln_w, ln_b, w_qk
   against a caller-held ``workspace``.  ``fixup_sum_limit`` > 0 lowers the weight-sum limit
   above which a (row, head) is recomputed by the exact two-pass softmax (0 = the default 2^100)."""
   _require_cuda(z, seq_mask, ln_w, ln_b, w_qkvgb, w_o, workspace)
-  _require(z.ndim == 3 and z.shape[0] == z.shape[1], f"triangle: z must be [N, N, C], got {tuple(z.shape)}")
+  if not (z.ndim == 3 and z.shape[0] == z.shape[1]):
+    raise ValueError(f"triangle: z must be [N, N, C], got {tuple(z.shape)}")
   N, _, Cn = z.shape
   HD = w_o.shape[1]
   _require(HD % num_head == 0, "triangle: output projection width not divisible by heads")
   D = HD // num_head
-  _require(tuple(w_qkvgb.shape) == (4 * HD + num_head, Cn), f"triangle: w_qkvgb shape {tuple(w_qkvgb.shape)}")
-  _require(tuple(w_o.shape) == (Cn, HD), f"triangle: w_o shape {tuple(w_o.shape)}")
+  if w_qkvgb.shape != (4 * HD + num_head, Cn):
+    raise ValueError(f"triangle: w_qkvgb shape {tuple(w_qkvgb.shape)}")
+  if w_o.shape != (Cn, HD):
+    raise ValueError(f"triangle: w_o shape {tuple(w_o.shape)}")
   _require(seq_mask.shape == (N,), "triangle: seq_mask must be [N]")
   zc = _bf16(z).contiguous()
   m8 = _u8(seq_mask).contiguous()
@@ -564,7 +570,8 @@ def triangle_multiplication(z: torch.Tensor, mask, w: dict, *, incoming: bool, a
   out = torch.empty_like(z3)
   lib = _lib.load()
   ws_bytes = int(lib.sf_hip_triangle_mult_workspace_bytes(N, Cn))
-  _require(ws_bytes > 0, f"triangle_multiplication: unsupported sizes N={N} C={Cn} (C must be 128)")
+  if ws_bytes <= 0:
+    raise ValueError(f"triangle_multiplication: unsupported sizes N={N} C={Cn} (C must be 128)")
   a = _lib.TriangleMultArgs()
   a.N, a.C, a.incoming, a.add_residual = N, Cn, int(bool(incoming)), int(bool(add_residual))
   m8 = _u8_or_none(mask)
