@@ -446,22 +446,29 @@ __global__ __launch_bounds__(64 * kPWaves) void tri_proj_kernel(const TriProjArg
   }
 }
 
-// The same for few positions: a block of 32 folded rows per workgroup (blockIdx.y) and an item per
-// wave, so that a small pair representation spreads over the chip.  One wave of the kernel above
+// The same for few positions (N <= 128): q, k, v or the bias per workgroup (blockIdx.y) and an item
+// per wave, so that a small pair representation spreads over the chip.  One wave of the kernel above
 // takes an item through all PB blocks in turn, and every workgroup first stages all of W: 14 us
-// whatever N, of which staging took 1.6, LayerNorm 0.9 and the blocks 9 (N = 20).
+// whatever N, of which staging took 1.6, LayerNorm 0.9 and the blocks 9 (N = 20).  Parts of one
+// block shorten that chain further but repeat the LayerNorm (1600 cycles a wave) and the loads of z:
+// C = 128, ending node, us, 4 parts / 13 parts / unsplit: N = 20 7.9 / 7.4 / 14.4, 64 9.2 / 10.1 / 15,
+// 128 10.8 / 16.4 / 16.
 constexpr int kSplitWaves = 4;
 
 template <int KC>
 __global__ __launch_bounds__(64 * kSplitWaves) void tri_proj_split_kernel(const TriProjArgs a) {
   using TD = TriDims<KC>;
   constexpr int C = TD::C, WP = TD::WP, NC = TD::NC, NB = TD::NB;
-  __shared__ __attribute__((aligned(16))) uint16_t sW[32 * WP];
-  __shared__ __attribute__((aligned(16))) float sOff[32];
+  __shared__ __attribute__((aligned(16))) uint16_t sW[C * WP];
+  __shared__ __attribute__((aligned(16))) float sOff[C];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, li = lane & 31;
-  const int N = a.N, nb = blockIdx.y;                   // 0 .. 3 NB - 1: q, k, v; 3 NB: bias
+  const int N = a.N, part = blockIdx.y;                 // 0, 1, 2, 3: q, k, v, bias
+  const bool bias = part == 3;
   const int bpr = a.NP / 32, item = blockIdx.x * kSplitWaves + wave;   // (a.items is a multiple of kSplitWaves)
+  // q, k, v of rows past N are not needed: the attention kernel computes row groups of 4 and stores
+  // rows below N only
+  if (!bias && blockIdx.x * kSplitWaves / bpr >= N) return;            // the workgroup's first row
   const int r = item / bpr, p0 = (item - r * bpr) * 32, p = p0 + li;
   const int za = a.transpose ? p : r, zb = a.transpose ? r : p;
   const bool valid = za < N && zb < N;
@@ -470,22 +477,30 @@ __global__ __launch_bounds__(64 * kSplitWaves) void tri_proj_split_kernel(const 
   u32x4 x[NC];
 #pragma unroll
   for (int kk = 0; kk < NC; ++kk) x[kk] = ld16(zp + 16 * kk);
-  const int src = nb < 3 * NB ? 32 * nb : 4 * C;        // first folded row of the block
-  constexpr int kStage = 32 * (C / 8) / (64 * kSplitWaves);
+  const int src = bias ? 4 * C : C * part, rows = bias ? 32 : C;         // folded rows of the part
+  constexpr int kStage = C * (C / 8) / (64 * kSplitWaves);
+  u32x4 wst[kStage];
+#pragma unroll
+  for (int j = 0; j < kStage; ++j) {
+    const int t = tid + j * 64 * kSplitWaves, n = min(t / (C / 8), rows - 1), c8 = (t % (C / 8)) * 8;
+    wst[j] = ld16(a.wf + (int64_t)(src + n) * C + c8);
+  }
 #pragma unroll
   for (int j = 0; j < kStage; ++j) {
     const int t = tid + j * 64 * kSplitWaves, n = t / (C / 8), c8 = (t % (C / 8)) * 8;
-    st16(&sW[n * WP + c8], ld16(a.wf + (int64_t)(src + n) * C + c8));
+    st16(&sW[n * WP + c8], wst[j]);
   }
-  if (tid < 32) sOff[tid] = a.off[src + tid];
+  if (tid < rows) sOff[tid] = a.off[src + tid];
   bf16x8 xo[NC];
   ln_operands<NC>(x, valid, xo);
   __syncthreads();
-  if (nb == 3 * NB) {                                   // uniform, as below
+  if (bias) {                                           // uniform, as below
     proj_bias_block<KC>(a, sW, sOff, 0, xo, (uint32_t)__ballot(sm != 0), r, p0, lane);
-  } else if (r < N) {   // (the attention kernel computes row groups of 4 and stores rows below N only)
-    if (nb < 2 * NB) proj_qk_block<KC>(a, nb / NB, nb % NB, sW, sOff, 0, xo, valid, r, p, lane);
-    else proj_v_block<KC>(a, nb - 2 * NB, sW, sOff, 0, xo, r, p0, lane);
+  } else if (r < N) {
+    for (int hh = 0; hh < NB; ++hh) {
+      if (part < 2) proj_qk_block<KC>(a, part, hh, sW, sOff, hh, xo, valid, r, p, lane);
+      else proj_v_block<KC>(a, hh, sW, sOff, hh, xo, r, p0, lane);
+    }
   }
 }
 
@@ -2128,7 +2143,7 @@ int triangle_fast(const sf_triangle_args* a, void* workspace, size_t workspace_b
     pa.q = ws.q; pa.k = ws.k; pa.vt = ws.vt; pa.bias = ws.bias;
     pa.items = NP * (NP / 32);
     if (pa.items <= kSplitItems) {
-      hipLaunchKernelGGL(tri_proj_split_kernel<KC>, dim3(pa.items / kSplitWaves, TD::ProjBlocks), dim3(64 * kSplitWaves), 0, st, pa);
+      hipLaunchKernelGGL(tri_proj_split_kernel<KC>, dim3(pa.items / kSplitWaves, 4), dim3(64 * kSplitWaves), 0, st, pa);
     } else {
       const int pgroups = persistent_groups(pa.items, &pa.items_per_wave);
       hipLaunchKernelGGL(tri_proj_kernel<KC>, dim3(pgroups), dim3(64 * kPWaves), 0, st, pa);

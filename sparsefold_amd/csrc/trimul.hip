@@ -189,36 +189,50 @@ __global__ __launch_bounds__(64 * kTW) void trimul_proj_kernel(const ProjArgs a)
   }
 }
 
-// The same for few positions: a block of 32 channels of one side per workgroup (blockIdx.y) and an
-// item per wave, so that a small pair representation spreads over the chip.  One wave of the kernel
-// above takes an item through all 8 blocks in turn, and every workgroup first stages all of W: 15 us
-// whatever N, of which staging took 1.6, LayerNorm 0.9 and the blocks 9 (N = 20).
+// The same for few positions (N <= 128): BPW blocks of 32 channels of one side per workgroup
+// (blockIdx.y) and an item per wave, so that a small pair representation spreads over the chip.  One
+// wave of the kernel above takes an item through all 8 blocks in turn, and every workgroup first
+// stages all of W: 15 us whatever N, of which staging took 1.6, LayerNorm 0.9 and the blocks 9
+// (N = 20).  More parts shorten that chain but repeat the LayerNorm (1600 cycles a wave) and the
+// loads of z.
 constexpr int kSplitWaves = 4;
 
+template <int BPW>
 __global__ __launch_bounds__(64 * kSplitWaves) void trimul_proj_split_kernel(const ProjArgs a) {
-  __shared__ __attribute__((aligned(16))) uint16_t sW[64 * kWS];     // 32 gate rows, 32 projection rows
-  __shared__ float sOff[64];
+  __shared__ __attribute__((aligned(16))) uint16_t sW[BPW * 64 * kWS];   // 32 BPW gate rows, then the projection rows
+  __shared__ float sOff[BPW * 64];
+  constexpr int G = 32 * BPW;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, li = lane & 31;
-  const int rg = 32 * blockIdx.y;                                    // first gate row: side kC + 32 nb
+  const int rg = G * blockIdx.y;                                     // first gate row: side kC + 32 nb
   const int item = blockIdx.x * kSplitWaves + wave;                  // (a.items is a multiple of kSplitWaves)
   u32x4 zn[8];
   bool ok;
   int R, col, m0, m1;
   load_item(a, item, li, half, zn, ok, R, col, m0, m1);
+  constexpr int kStage = 2 * G * (kC / 8) / (64 * kSplitWaves);
+  u32x4 wst[kStage];
 #pragma unroll
-  for (int j = 0; j < 64 * (kC / 8) / (64 * kSplitWaves); ++j) {
+  for (int j = 0; j < kStage; ++j) {
     const int t = tid + j * 64 * kSplitWaves, n = t >> 4, c8 = (t & 15) * 8;
-    st16(&sW[n * kWS + c8], ld16(a.w + (int64_t)((n >> 5) * 2 * kC + rg + (n & 31)) * kC + c8));
+    wst[j] = ld16(a.w + (int64_t)((n / G) * 2 * kC + rg + n % G) * kC + c8);
   }
-  if (tid < 64) sOff[tid] = a.off[(tid >> 5) * 2 * kC + rg + (tid & 31)];
+#pragma unroll
+  for (int j = 0; j < kStage; ++j) {
+    const int t = tid + j * 64 * kSplitWaves, n = t >> 4, c8 = (t & 15) * 8;
+    st16(&sW[n * kWS + c8], wst[j]);
+  }
+  if (tid < 2 * G) sOff[tid] = a.off[(tid / G) * 2 * kC + rg + tid % G];
   bf16x8 xo[8];
   ln128_operands(zn, ok, xo);
   __syncthreads();
   const int64_t pstride = (int64_t)a.Pn * a.Pn;
   char* dstp = reinterpret_cast<char*>(rg >= kC ? a.b : a.a) + (int64_t)(rg & (kC - 1)) * pstride * 2;
-  proj_block(sW, sW + 32 * kWS, sOff, sOff + 32, xo, ok && m0 != 0 && m1 != 0, dstp, pstride,
-             (4 * half * pstride + (int64_t)R * a.Pn + col) * 2, lane);
+  const bool keep = ok && m0 != 0 && m1 != 0;
+  const int64_t lofs = (4 * half * pstride + (int64_t)R * a.Pn + col) * 2;
+  for (int j = 0; j < BPW; ++j)
+    proj_block(sW + 32 * j * kWS, sW + (G + 32 * j) * kWS, sOff + 32 * j, sOff + G + 32 * j, xo, keep,
+               dstp + 32 * j * pstride * 2, pstride, lofs, lane);
 }
 
 struct OutArgs {
@@ -560,7 +574,10 @@ extern "C" int sf_hip_triangle_mult_fwd(const sf_triangle_mult_args* a, void* wo
     pa.w = w.wglu; pa.off = w.oglu; pa.a = w.a; pa.b = w.b;
     pa.items = Pn * (Pn / 32);                          // every plane row, padding included
     if (pa.items <= kSplitItems) {
-      hipLaunchKernelGGL(trimul_proj_split_kernel, dim3(pa.items / kSplitWaves, 8), dim3(64 * kSplitWaves), 0, st, pa);
+      // a block per workgroup while the waves fill one per SIMD: N = 64 (128 items) 5.8 us against 6.8
+      // for two blocks; N = 128 (512 items) 14.2 against 11.9
+      if (pa.items <= 128) hipLaunchKernelGGL(trimul_proj_split_kernel<1>, dim3(pa.items / kSplitWaves, 8), dim3(64 * kSplitWaves), 0, st, pa);
+      else hipLaunchKernelGGL(trimul_proj_split_kernel<2>, dim3(pa.items / kSplitWaves, 4), dim3(64 * kSplitWaves), 0, st, pa);
     } else {
       const int waves = launch_grid(reinterpret_cast<const void*>(trimul_proj_kernel), pa.items);
       pa.items_per_wave = (pa.items + waves - 1) / waves;
