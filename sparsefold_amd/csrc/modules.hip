@@ -119,10 +119,15 @@ struct CondTermsArgs {
 };
 constexpr int kCondMaxCs = 384;
 
-__global__ __launch_bounds__(256) void cond_terms_kernel(const CondTermsArgs a) {
+// CS: the condition width, known when compiled (kCondMaxCs), or 0: any allowed one.  With the tests
+// for the width's end in the unrolled loads and MFMAs, every load sat in a branch of its own (the
+// first one waited for at once), every MFMA waited for its LDS reads alone, and the kernel took 260
+// registers: one workgroup per CU, so that the 288 of 1024 x 384 -> 768 ran in two rounds: 21.4 us, now 13.8.
+template <int CS>
+__global__ __launch_bounds__(256, CS ? 2 : 1) void cond_terms_kernel(const CondTermsArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint16_t sA[];   // [64][Cs + 8], then lnc_w, lnc_b (f32)
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5, li = lane & 31;
-  const int Cs = a.Cs, pitch = Cs + 8, nch = Cs / 8;
+  const int Cs = CS ? CS : a.Cs, pitch = Cs + 8, nch = Cs / 8;
   const int term = blockIdx.z;                                  // 0 scale, 1 shift, 2 zgate
   const int64_t r0 = (int64_t)blockIdx.x * 64;
   const int n0 = blockIdx.y * 128;
@@ -155,9 +160,8 @@ __global__ __launch_bounds__(256) void cond_terms_kernel(const CondTermsArgs a) 
     }
   __syncthreads();
   {
-    float mean = 0.f, rstd = 1.f;
     if (term < 2) {
-      float sum = 0.f;
+      float mean, rstd, sum = 0.f;
 #pragma unroll
       for (int t = 0; t < kChunks; ++t)
 #pragma unroll
@@ -179,25 +183,31 @@ __global__ __launch_bounds__(256) void cond_terms_kernel(const CondTermsArgs a) 
       sq += __shfl_xor(sq, 1);
       sq += __shfl_xor(sq, 2);
       rstd = rsqrtf(sq / (float)Cs + 1e-5f);
-    }
 #pragma unroll
-    for (int t = 0; t < kChunks; ++t) {
-      const int ch = q + kParts * t;
-      if (ch >= nch) continue;
-      u32x4 y = v[t];
-      if (term < 2) {
+      for (int t = 0; t < kChunks; ++t) {
+        const int ch = q + kParts * t;
+        if (ch >= nch) continue;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int c = 8 * ch + 2 * e;
-          y[e] = pack_bf2((bflo(v[t][e]) - mean) * rstd * sG[c] + sB[c],
-                          (bfhi(v[t][e]) - mean) * rstd * sG[c + 1] + sB[c + 1]);
+          v[t][e] = pack_bf2((bflo(v[t][e]) - mean) * rstd * sG[c] + sB[c],
+                             (bfhi(v[t][e]) - mean) * rstd * sG[c + 1] + sB[c + 1]);
         }
       }
-      st16(&sA[rr * pitch + 8 * ch], y);
     }
+#pragma unroll
+    for (int t = 0; t < kChunks; ++t)
+      if (q + kParts * t < nch) st16(&sA[rr * pitch + 8 * (q + kParts * t)], v[t]);
   }
   __syncthreads();
   const float* bias = term == 0 ? a.b_scale : term == 1 ? nullptr : a.b_zc;
+  // the bias loads' latency passes under the products; without a bias, any C floats (no branches)
+  const float* bp = bias ? bias : reinterpret_cast<const float*>(W);
+  float bn[4][4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) bn[j][e] = bp[nq + 8 * j + 4 * half + e];
   f32x16 acc[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -210,11 +220,6 @@ __global__ __launch_bounds__(256) void cond_terms_kernel(const CondTermsArgs a) 
       for (int i = 0; i < 2; ++i)                             // rows 32 i + li: two independent chains
         acc[i] = mfma32(as_bf16x8(wr[kc]), as_bf16x8(ld16(sA + (32 * i + li) * pitch + 8 * half + 16 * kc)), acc[i]);
     }
-  float bn[4][4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) bn[j][e] = bias ? bias[nq + 8 * j + 4 * half + e] : 0.f;
   uint16_t* outb = term == 0 ? a.scale : term == 1 ? a.shift : a.zgate;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -227,7 +232,7 @@ __global__ __launch_bounds__(256) void cond_terms_kernel(const CondTermsArgs a) 
       float v4[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        v4[e] = acc[i][4 * j + e] + bn[j][e];
+        v4[e] = acc[i][4 * j + e] + (bias ? bn[j][e] : 0.f);
         if (term != 1) v4[e] = sigmoidf_(v4[e]);
       }
       *reinterpret_cast<u32x2*>(out + n) = u32x2{pack_bf2(v4[0], v4[1]), pack_bf2(v4[2], v4[3])};
@@ -251,7 +256,9 @@ int cond_terms(int64_t rows, int C, int Cs, const void* cond, const float* lnc_w
   t.w_zc = static_cast<const uint16_t*>(w_zc); t.b_scale = b_scale; t.b_zc = b_zc;
   t.scale = static_cast<uint16_t*>(scale); t.shift = static_cast<uint16_t*>(shift); t.zgate = static_cast<uint16_t*>(zgate);
   const size_t lds = (size_t)64 * (Cs + 8) * 2 + (size_t)2 * Cs * 4;   // 53 KB at Cs = 384
-  hipLaunchKernelGGL(cond_terms_kernel, dim3((unsigned)((rows + 63) / 64), (unsigned)(C / 128), 3), dim3(256), lds, st, t);
+  const dim3 grid((unsigned)((rows + 63) / 64), (unsigned)(C / 128), 3);
+  if (Cs == kCondMaxCs) hipLaunchKernelGGL(cond_terms_kernel<kCondMaxCs>, grid, dim3(256), lds, st, t);
+  else hipLaunchKernelGGL(cond_terms_kernel<0>, grid, dim3(256), lds, st, t);
   return sf_check_launch("cond_terms_kernel");
 }
 
