@@ -768,8 +768,11 @@ int route(const sf_attention_args* a, bool allow_split, AttnRoute& r) {
   r.attn2 = r.vec;
   r.ksplit = 1;
   r.pl = Attn2Plan{};
-  if (a->kv_index != nullptr && (!r.attn2 || a->kv_zero_row < 0)) {
-    sf_set_error("attention: gathered K/V rows need 16-byte aligned q/k/v rows and strides and kv_zero_row >= 0");
+  bool bias8 = a->bias == nullptr || aligned8(a->bias);
+  for (int s = 0; s < 4 && bias8 && a->bias != nullptr; ++s) bias8 = a->bias_s[s] % 4 == 0;
+  if (a->kv_index != nullptr && (!r.attn2 || !bias8 || a->kv_zero_row < 0)) {
+    sf_set_error("attention: gathered K/V rows need 16-byte aligned q/k/v rows and strides, an 8-byte aligned "
+                 "bias and kv_zero_row >= 0");
     return 1;
   }
   if (!r.attn2) return 0;
