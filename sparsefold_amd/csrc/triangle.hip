@@ -173,7 +173,29 @@ struct TriFoldArgs {
   // the attention rows worth computing: row groups (4 rows) with a row r < N and seq[r] != 0,
   // listed in rgl[1..count], count in rgl[0] (null: no list)
   int* rgl; int rg, N; const uint8_t* seq;
+  // bias of the attention rows past N (the projection runs the rows below N only)
+  uint16_t* bias; int NP, H, transpose;
 };
+
+// The bias of attention rows N .. NP - 1, which the projection does not visit, in 16-byte pieces of 8
+// stored keys: -inf for a key past N, 0 for a valid key of a padding query.  Starting node: the
+// padding queries' rows.  Ending node: every query's tiles of 64 keys that hold a key past N (their
+// valid keys are written by the projection afterwards).
+__device__ __forceinline__ void fill_padding_bias(const TriFoldArgs& a, int idx, int stride) {
+  const int N = a.N, NP = a.NP;
+  const int q0 = a.transpose ? 0 : N, pc0 = a.transpose ? (N >> 6) * 8 : 0;   // first query, first piece
+  const int pcs = NP / 8 - pc0, per_h = (NP - q0) * pcs;
+  for (int f = idx; f < a.H * per_h; f += stride) {
+    const int h = f / per_h, rest = f - h * per_h, js = 8 * (pc0 + rest % pcs), i = q0 + rest / pcs;
+    uint32_t w[4];
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) {                         // stored position -> key (bias_pos64 inverted)
+      const int s0 = (js & 63) + e, j = (js & ~63) + (s0 & 32) + 8 * ((s0 >> 2) & 3) + 4 * ((s0 >> 4) & 1) + (s0 & 3);
+      w[e / 2] = pack_bf2(j >= N ? -INFINITY : 0.f, j + 1 >= N ? -INFINITY : 0.f);
+    }
+    st16(a.bias + bias_off_stored(h, i, js, NP), u32x4{w[0], w[1], w[2], w[3]});
+  }
+}
 
 template <int KC>
 __global__ __launch_bounds__(256) void tri_fold_kernel(const TriFoldArgs a) {
@@ -207,6 +229,7 @@ __global__ __launch_bounds__(256) void tri_fold_kernel(const TriFoldArgs a) {
     return;
   }
   const int zstride = (gridDim.x - 1) * blockDim.x;         // the folding workgroups clear the flags
+  if (a.N != a.NP) fill_padding_bias(a, blockIdx.x * blockDim.x + threadIdx.x, zstride);
   for (int f = blockIdx.x * blockDim.x + threadIdx.x; f < a.nflags; f += zstride) a.flags[f] = 0;
   for (int f = blockIdx.x * blockDim.x + threadIdx.x; f < a.nctr; f += zstride) a.ctr[f] = 0;
   for (int f = blockIdx.x * blockDim.x + threadIdx.x; f < a.ndefer; f += zstride) a.defer[f] = 0;
@@ -241,7 +264,7 @@ struct TriProjArgs {
   const uint16_t* z; const uint8_t* seq;
   const uint16_t* wf; const float* off;   // folded weight [Cols, C] and column offsets
   uint16_t *q, *k, *vt, *bias;
-  int items, items_per_wave;          // items = NP * NP / 32 position blocks
+  int items, items_per_wave;          // items = N * NP / 32 position blocks
 };
 
 // One block of 32 folded projection rows (rows 32 nb .. of sW, offsets sOff) of 32 positions p0 + li
@@ -466,9 +489,6 @@ __global__ __launch_bounds__(64 * kSplitWaves) void tri_proj_split_kernel(const 
   const int N = a.N, part = blockIdx.y;                 // 0, 1, 2, 3: q, k, v, bias
   const bool bias = part == 3;
   const int bpr = a.NP / 32, item = blockIdx.x * kSplitWaves + wave;   // (a.items is a multiple of kSplitWaves)
-  // q, k, v of rows past N are not needed: the attention kernel computes row groups of 4 and stores
-  // rows below N only
-  if (!bias && blockIdx.x * kSplitWaves / bpr >= N) return;            // the workgroup's first row
   const int r = item / bpr, p0 = (item - r * bpr) * 32, p = p0 + li;
   const int za = a.transpose ? p : r, zb = a.transpose ? r : p;
   const bool valid = za < N && zb < N;
@@ -496,7 +516,7 @@ __global__ __launch_bounds__(64 * kSplitWaves) void tri_proj_split_kernel(const 
   __syncthreads();
   if (bias) {                                           // uniform, as below
     proj_bias_block<KC>(a, sW, sOff, 0, xo, (uint32_t)__ballot(sm != 0), r, p0, lane);
-  } else if (r < N) {
+  } else {
     for (int hh = 0; hh < NB; ++hh) {
       if (part < 2) proj_qk_block<KC>(a, part, hh, sW, sOff, hh, xo, valid, r, p, lane);
       else proj_v_block<KC>(a, hh, sW, sOff, hh, xo, r, p0, lane);
@@ -2132,6 +2152,7 @@ int triangle_fast(const sf_triangle_args* a, void* workspace, size_t workspace_b
     fa.ctr = ws.ctr; fa.nctr = ws.nctr;
     fa.defer = ws.defer; fa.ndefer = N;
     fa.rgl = ws.rgl; fa.rg = NP / 4; fa.N = N; fa.seq = a->seq_mask;
+    fa.bias = ws.bias; fa.NP = NP; fa.H = H; fa.transpose = a->transpose;
     hipLaunchKernelGGL(tri_fold_kernel<KC>, dim3(TD::Cols / 4 + 1), dim3(256), 0, st, fa);
     if (int rc = sf_check_launch("tri_fold_kernel")) return rc;
 
@@ -2141,7 +2162,9 @@ int triangle_fast(const sf_triangle_args* a, void* workspace, size_t workspace_b
     pa.z = (const uint16_t*)a->z; pa.seq = a->seq_mask;
     pa.wf = ws.wf; pa.off = ws.off;
     pa.q = ws.q; pa.k = ws.k; pa.vt = ws.vt; pa.bias = ws.bias;
-    pa.items = NP * (NP / 32);
+    // rows below N: q, k, v of the others are not needed (the attention kernel stores rows below N
+    // only), and their bias is filled in by the fold kernel
+    pa.items = N * (NP / 32);
     if (pa.items <= kSplitItems) {
       hipLaunchKernelGGL(tri_proj_split_kernel<KC>, dim3(pa.items / kSplitWaves, 4), dim3(64 * kSplitWaves), 0, st, pa);
     } else {
