@@ -200,15 +200,15 @@ __global__ __launch_bounds__(256) void attention_fwd_kernel(const sf_attention_a
 }
 
 // ---------------------------------------------------------------------------------------
-// Direct-to-LDS form (16-byte aligned q/k/v rows, head dims multiple of 8, bias rows 8-byte
-// aligned).  A wave owns 32 queries of one (batch, head).  Keys stream in tiles of 64:
+// Direct-to-LDS form (16-byte aligned q/k/v rows, head dims multiple of 8; bias rows of any
+// alignment).  A wave owns 32 queries of one (batch, head).  Keys stream in tiles of 64:
 //   K, V  copied row-major into LDS by global_load_lds_dwordx4 (1 KB per instruction; the
 //         16-byte pieces of a K row are XOR-swizzled by key so that the S^T operand reads of
 //         consecutive lanes hit distinct banks)
-//   S^T   = K Q^T (+ bias tile as the fp32 accumulator seed, + one MFMA k-step that adds the
-//         key-mask column: 0, SF_MASKED_LOGIT for masked keys, kPadKey for keys past K)
-//   P     = exp(scale (S^T - m)) with the running row maximum m of S^T = q.k + bias / scale
-//         (the scale is applied in fp32); lane half h holds keys 8c + 4h + e of each 32-key half
+//   S^T   = K Q^T
+//   P     = 2^(t - m) of the fp32 logits t = scale log2(e) S^T + log2(e) bias, with m near the row's
+//         maximum; masked keys have t = SF_MASKED_LOGIT and keys past K weigh 0; lane half h holds
+//         keys 8c + 4h + e of each 32-key half
 //   O^T  += V^T P^T, the V^T operand read straight from the row-major V tile with
 //         ds_read_b64_tr_b16: lane (d, h) of 16-lane group G gets the 4 keys the matching P^T
 //         lane holds, for one dim -- no transposed copy of V is ever made.
@@ -221,7 +221,6 @@ typedef __attribute__((address_space(3))) uint32_t lds_u32a;
 typedef short v4i16 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
 
-constexpr float kPadKey = -8.507059173023462e37f;  // -2^126: keys past K, below any masked key
 constexpr float kMassLimit = 1.152921504606846976e18f;   // 2^60: weight mass of a tile that moves m
 
 struct Attn2Plan {
@@ -276,8 +275,9 @@ __device__ __forceinline__ u32x4 shift_down8(u32x4 w, int s) {
 // BL = 2: the same tile and layout for rows of any alignment and any K >= 8, loaded 16 bytes a lane
 // into registers a tile ahead (direct-to-LDS copies need aligned rows) and written to LDS at the
 // tile's start.  BL = 0: each lane loads its keys from global memory.
+// Three waves per SIMD are asked for where LDS holds them and 168 registers reach.
 template <int DP, bool SHARED, int KC, int BL>
-__global__ __launch_bounds__(256) void attn2_kernel(const sf_attention_args a, const Attn2Plan pl) {
+__global__ __launch_bounds__(256, SHARED && (DP == 32 || (KC <= 3 && BL < 2)) ? 3 : 1) void attn2_kernel(const sf_attention_args a, const Attn2Plan pl) {
   using T = Attn2Tile<DP>;
   constexpr int kWaveBufs = SHARED ? 1 : 4;                 // tile sets in LDS (shared or per wave)
   constexpr int kKVRegion = kWaveBufs * 2 * T::kBufBytes;
@@ -337,14 +337,14 @@ __global__ __launch_bounds__(256) void attn2_kernel(const sf_attention_args a, c
   if (a.mask_q && i < Q) qvalid = a.mask_q[b0 * a.mq_s[0] + b1 * a.mq_s[1] + (int64_t)i * a.mq_s[2]] != 0;
   const bool any_qmasked = __any(!qvalid && i < Q);          // uniform
 
-  // ---- Q operand (unscaled: S^T holds q.k + bias / scale, scaled in fp32 at the exp) ----
+  // ---- Q operand (unscaled: S^T holds q.k, scaled in fp32) ----
   bf16x8 qb[DP / 16];
 #pragma unroll
   for (int kk = 0; kk < DP / 16; ++kk) {
     const int d0 = 16 * kk + 8 * half;
     qb[kk] = as_bf16x8(d0 < D ? ld16(qp + (int64_t)iq * a.q_s[2] + d0) : u32x4{0, 0, 0, 0});
   }
-  const float cs = a.scale * SF_LOG2E, inv_scale = 1.0f / a.scale;
+  const float cs = a.scale * SF_LOG2E;
 
   // ---- tile copy: chunk c of a tile, K chunks first ----
   uint8_t* wsm = smem + (SHARED ? 0 : wave * 2 * T::kBufBytes);
@@ -470,10 +470,7 @@ __global__ __launch_bounds__(256) void attn2_kernel(const sf_attention_args a, c
   for (int db = 0; db < DP / 32; ++db)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[db][r] = 0.f;
-  float m = -INFINITY, l = 0.f;
-  bf16x8 ones_b;                                             // B operand: 1 at k = 0 (half 0)
-#pragma unroll
-  for (int e = 0; e < 8; ++e) ones_b[e] = (__bf16)((e == 0 && half == 0) ? 1.0f : 0.0f);
+  float m = -3.402823466e38f, l = 0.f;                       // the lowest float: m stays finite
 
   // Waits: the copies into LDS are ordinary loads to the compiler, so every wait is followed
   // by a compiler barrier (or __syncthreads) that keeps the LDS reads of the tile after it.
@@ -513,46 +510,61 @@ __global__ __launch_bounds__(256) void attn2_kernel(const sf_attention_args a, c
       load_side(j0 + 64);
     }
     if (wactive) {
-      // ---- S^T = K Q^T + bias (+ mask column) ----
-      const bool need_mask = mbits != ~0ull;                 // uniform
+      // ---- logits s = scale log2(e) (S^T = K Q^T) + log2(e) bias; register r of half kb is key
+      //      32 kb + 8 (r / 4) + 4 half + r % 4 of the tile.  A masked key's is SF_MASKED_LOGIT
+      //      whatever its q.k and bias are (NaN included), a key's past K is -inf; a masked query
+      //      masks every key.  They are rounded before m is subtracted: in one fma with -m, what the
+      //      rounding of a large m had lost (2^103 at a bias of 2e38) became the difference. ----
       f32x16 s[2];
+      auto logits = [&]() __attribute__((always_inline)) {
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
+        for (int kb = 0; kb < 2; ++kb) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
+          for (int r = 0; r < 16; ++r) s[kb][r] = 0.f;
+          const int key = 32 * kb + li;
 #pragma unroll
-          for (int e = 0; e < 2; ++e) {
-            s[kb][4 * c + 2 * e] = bflo(bcur[4 * kb + c][e]) * inv_scale;
-            s[kb][4 * c + 2 * e + 1] = bfhi(bcur[4 * kb + c][e]) * inv_scale;
+          for (int kk = 0; kk < KC; ++kk) {                  // chunks past D are zeros in q
+            const int piece = (2 * kk + half) ^ T::kswz(key);
+            s[kb] = mfma32(as_bf16x8(ld16(kt + key * T::kRowBytes + piece * 16)), qb[kk], s[kb]);
           }
-        const int key = 32 * kb + li;
-#pragma unroll
-        for (int kk = 0; kk < KC; ++kk) {                    // chunks past D are zeros in q
-          const int piece = (2 * kk + half) ^ T::kswz(key);
-          s[kb] = mfma32(as_bf16x8(ld16(kt + key * T::kRowBytes + piece * 16)), qb[kk], s[kb]);
         }
-        if (need_mask) {
-          bf16x8 mc;
 #pragma unroll
-          for (int e = 0; e < 8; ++e) mc[e] = (__bf16)0.0f;
-          const float mv = ((mbits >> key) & 1ull) ? 0.0f : (j0 + key < K ? SF_MASKED_LOGIT : kPadKey);
-          mc[0] = (__bf16)(half == 0 ? mv : 0.0f);
-          s[kb] = mfma32(mc, ones_b, s[kb]);
+        for (int kb = 0; kb < 2; ++kb) {
+          // the bias stays packed until S^T is there (unpacked ahead of it, it took 32 registers more)
+          asm volatile("" : "+v"(s[kb]), "+v"(bcur[4 * kb]), "+v"(bcur[4 * kb + 1]), "+v"(bcur[4 * kb + 2]), "+v"(bcur[4 * kb + 3]));
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const uint32_t w = bcur[4 * kb + (r >> 2)][(r >> 1) & 1];
+            s[kb][r] = __builtin_fmaf(s[kb][r], cs, ((r & 1) ? bfhi(w) : bflo(w)) * SF_LOG2E);
+          }
         }
-      }
-      if (any_qmasked && !qvalid) {                          // masked query: uniform over keys < K
+        if (mbits != ~0ull || any_qmasked) {                 // uniform
+          // s = other where the key's bit is clear: bit 8 (r / 4) + r % 4 of its half's word
+          auto replace = [&](uint64_t keys, bool lane_ok, float other) __attribute__((always_inline)) {
+            asm volatile("" : "+s"(keys));                   // (opaque: masks formed ahead of the branch cost 30%)
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
+            for (int kb = 0; kb < 2; ++kb) {
+              const uint32_t w = lane_ok ? (uint32_t)(keys >> (32 * kb)) >> (4 * half) : 0u;
 #pragma unroll
-          for (int r = 0; r < 16; ++r)
-            s[kb][r] = j0 + 32 * kb + 8 * (r >> 2) + 4 * half + (r & 3) < K ? 0.0f : kPadKey;
-      }
-      // ---- softmax against a reference point m (in units of S^T) ----
-      // Tile 0 sets m to the row maximum of its 64 keys.  Later tiles keep it unless the
+              for (int r = 0; r < 16; ++r) {
+                uint32_t keep;                               // all ones or none (from C, a compare and a select)
+                asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(keep) : "v"(w), "n"(8 * (r >> 2) + (r & 3)));
+                s[kb][r] = __uint_as_float((__float_as_uint(s[kb][r]) & keep) | (__float_as_uint(other) & ~keep));
+              }
+            }
+          };
+          const uint64_t below = j0 + 64 <= K ? ~0ull : ~0ull >> (j0 + 64 - K);   // keys below K
+          if (mbits != below || any_qmasked) replace(mbits, qvalid, SF_MASKED_LOGIT);
+          if (below != ~0ull) replace(below, true, -INFINITY);
+        }
+      };
+      // ---- softmax against a reference point m (log2 units) ----
+      // The first tile sets m to the row maximum of its 64 keys.  Later tiles keep it unless the
       // probability mass of the tile exceeds kMassLimit (all weights are >= 0, so the sum bounds
       // every weight and an overflow cannot pass unnoticed); then m moves to the tile's maximum
       // and what is accumulated is rescaled.  This replaces a running maximum (a max over the
-      // tile, one exp and a rescale of O every tile) by one compare.
+      // tile, one exp and a rescale of O every tile) by one compare.  m stays finite, so that a
+      // tile of -inf logits weighs nothing.
       auto row_max = [&]() __attribute__((always_inline)) {
         float v = s[0][0];
 #pragma unroll
@@ -561,32 +573,42 @@ __global__ __launch_bounds__(256) void attn2_kernel(const sf_attention_args a, c
           for (int r = 0; r < 16; ++r) v = fmaxf(v, s[kb][r]);
         return fmaxf(v, __shfl_xor(v, 32));
       };
-      auto weights = [&](float mref, bf16x2 (&pw)[16]) __attribute__((always_inline)) {
-        const float mb = mref * cs;
+      auto subtract = [&](float mref) __attribute__((always_inline)) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) s[kb][r] -= mref;
+      };
+      auto weights = [&](bf16x2 (&pw)[16]) __attribute__((always_inline)) {
         float t0 = 0.f, t1 = 0.f;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
-            pw[8 * kb + e] = cvt_bf2(fast_exp2(__builtin_fmaf(s[kb][2 * e], cs, -mb)),
-                                     fast_exp2(__builtin_fmaf(s[kb][2 * e + 1], cs, -mb)));
+            pw[8 * kb + e] = cvt_bf2(fast_exp2(s[kb][2 * e]), fast_exp2(s[kb][2 * e + 1]));
             if (e & 1) t1 = add_bf2(pw[8 * kb + e], t1); else t0 = add_bf2(pw[8 * kb + e], t0);
           }
         return t0 + t1;
       };
-      if (t == t_begin) m = row_max();
       bf16x2 pw[16];
-      float ts = weights(m, pw);
-      if (__any(!(ts <= kMassLimit))) {                      // rare: move m up and rescale
-        const float mnew = fmaxf(m, row_max());
-        const float alpha = fast_exp2((m - mnew) * cs);
-        m = mnew;
-        l *= alpha;
+      float ts;
+      // the first tile, and a tile whose mass is too large (its logits are formed again: kept to that
+      // point they cost a wave per SIMD)
+      for (bool raise = t == t_begin;; raise = true) {
+        logits();
+        if (raise) {
+          const float mnew = fmaxf(m, row_max());
+          const float alpha = fast_exp2(m - mnew);
+          m = mnew;
+          l *= alpha;
 #pragma unroll
-        for (int db = 0; db < DP / 32; ++db)
+          for (int db = 0; db < DP / 32; ++db)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
-        ts = weights(m, pw);
+            for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
+        }
+        subtract(m);
+        ts = weights(pw);
+        if (raise || !__any(!(ts <= kMassLimit))) break;
       }
       l += ts;
       // ---- O^T += V^T P^T ----
@@ -675,7 +697,7 @@ __global__ __launch_bounds__(256) void attn2_kernel(const sf_attention_args a, c
 
 // Combine of the key-range slices: thread per (query block, query, 4 dims).  O and l of each
 // slice are relative to the slice's own reference point m_s; with M = max m_s the result is
-// sum_s O_s 2^(cs (m_s - M)) / sum_s l_s 2^(cs (m_s - M)), then the gate.  All loads of a thread
+// sum_s O_s 2^(m_s - M) / sum_s l_s 2^(m_s - M), then the gate.  All loads of a thread
 // are independent and issued together: one memory round trip per thread.
 template <int DP, int KS>
 __global__ __launch_bounds__(256) void attn2_combine_kernel(const sf_attention_args a, const Attn2Plan pl) {
@@ -697,7 +719,6 @@ __global__ __launch_bounds__(256) void attn2_combine_kernel(const sf_attention_a
   }
   const int i = qblk * 32 + li;
   if (i >= a.Q || d0 >= a.Dv) return;
-  const float cs = a.scale * SF_LOG2E;
   const float* base = pl.part + blk * KS * 32 * (DP + 2);
   f32x2 ml[KS];
   f32x4 os[KS];
@@ -712,7 +733,7 @@ __global__ __launch_bounds__(256) void attn2_combine_kernel(const sf_attention_a
   float lsum = 0.f, v[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int sl = 0; sl < KS; ++sl) {
-    const float w = fast_exp2((ml[sl][0] - mx) * cs);
+    const float w = fast_exp2(ml[sl][0] - mx);
     lsum += w * ml[sl][1];
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] += w * os[sl][e];
