@@ -603,7 +603,7 @@ static int self_attention_run(const sf_self_attention_args* a, void* workspace, 
   if ((rc = sf_attention_run(&t, split_ws, split, st))) return rc;
   return zero_init_out(rows, a->C, HD, o, pre || fused_cond ? nullptr : a->cond, a->N, a->Cs, a->w_zc, a->b_zc,
                        a->w_t2, a->add_residual ? a->x : nullptr, a->out, ws, st,
-                       pre ? a->pre_zgate : c_zgate, pre ? a->pre_rs : a->C);
+                       pre ? a->pre_zgate : fused_cond ? c_zgate : nullptr, pre ? a->pre_rs : a->C);
 }
 
 extern "C" int sf_hip_self_attention_fwd(const sf_self_attention_args* a, void* workspace,
@@ -1141,7 +1141,7 @@ extern "C" int sf_hip_transition_fwd(const sf_transition_args* a, void* workspac
   if ((rc = sf_hip_linear_fwd(&g, st))) return rc;
   return zero_init_out(rows, a->C, a->I, c, pre || fused_cond ? nullptr : a->cond, a->N, a->Cs, a->w_zc, a->b_zc,
                        a->w2, a->add_residual ? a->x : nullptr, a->out, ws, st,
-                       pre ? a->pre_zgate : c_zgate, pre ? a->pre_rs : a->C);
+                       pre ? a->pre_zgate : fused_cond ? c_zgate : nullptr, pre ? a->pre_rs : a->C);
 }
 
 namespace {
