@@ -147,6 +147,9 @@ typedef struct sf_linear_args {
 } sf_linear_args;
 
 int sf_hip_linear_fwd(const sf_linear_args* a, void* stream);
+/* Whether sf_hip_linear_fwd runs `a` (arguments it accepts) on its kernel of 256 x 256 tiles: 1 or 0.
+ * Host only; nothing is launched or dereferenced. */
+int sf_hip_linear_large_tiles(const sf_linear_args* a);
 
 /* ---------------------------------------------------------------------------------------
  * Triangle attention, starting (transpose = 0) or ending (transpose = 1) node, whole module:

@@ -177,6 +177,7 @@ SIGNATURES = [
     ("sf_hip_attention_fwd", C.c_int, [C.POINTER(AttentionArgs), _vp]),
     ("sf_hip_layer_norm_fwd", C.c_int, [C.POINTER(LayerNormArgs), _vp]),
     ("sf_hip_linear_fwd", C.c_int, [C.POINTER(LinearArgs), _vp]),
+    ("sf_hip_linear_large_tiles", C.c_int, [C.POINTER(LinearArgs)]),
     ("sf_hip_triangle_workspace_bytes", C.c_size_t, [_i32, _i32, _i32, _i32]),
     ("sf_hip_triangle_attn_fwd", C.c_int, [C.POINTER(TriangleArgs), _vp, C.c_size_t, _vp]),
     ("sf_hip_triangle_stage_fwd", C.c_int, [C.POINTER(TriangleArgs), _i32, _vp, C.c_size_t, _vp]),

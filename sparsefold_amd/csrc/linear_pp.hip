@@ -24,9 +24,9 @@
 // pieces and are read back in the accumulator's layout, the results go out as whole rows.  (fp32
 // tiles through LDS and a barrier, as in linear64_kernel, cost 6 to 8 us per 256 x 256 tile.)
 //
-// Measured against linear64_kernel (random bf16 data, us a call): 8192 x 8192 x 1024 129 against 163,
-// 5120 x 3072 x 768 33 against 38, 3700 x 3072 x 768 27 against 34, 128 batched 768^3 (with the
-// triangle multiplication around them) 407 against 453.  What is left at 5120 x 3072 x 768: 7 us of
+// Measured against linear64_kernel (random bf16 data, us a call): 8192 x 8192 x 1024 134 against 174,
+// 5120 x 3072 x 768 32 against 38, 3700 x 3072 x 768 27 against 35, 128 batched 768^3 148 against 196
+// (the triangle multiplication around them 412 against 464).  What is left at 5120 x 3072 x 768: 7 us of
 // launch, first copies and barriers, 5 us of result stores at the memory's write rate, 18 us of
 // MFMAs at the clock the matrix cores hold on random data.
 #include <algorithm>
@@ -358,6 +358,14 @@ int64_t tiles(const sf_linear_args* a, int side) {
   return ((a->M + side - 1) / side) * (((int64_t)a->N + side - 1) / side) * (a->batch > 1 ? a->batch : 1);
 }
 
+// Workgroups of a launch: as many as are resident at once, a multiple of 8 (XCDs).  256 where no device
+// is there to ask (the host-only query).
+int64_t workgroups(const sf_linear_args* a) {
+  const void* kernel = a->glu ? reinterpret_cast<const void*>(linear_pp_kernel<true>) : reinterpret_cast<const void*>(linear_pp_kernel<false>);
+  const int n = sf_resident_workgroups(kernel, 512) / 8 * 8;
+  return n > 0 ? n : 256;
+}
+
 // bytes [p, p + ((rows - 1) rs + n) * 2) of a row-strided bf16 operand (rs > 0) meet y's
 bool meets_y(const sf_linear_args* a, const void* p, int64_t rows, int64_t rs) {
   const uintptr_t p0 = reinterpret_cast<uintptr_t>(p), p1 = p0 + ((rows - 1) * rs + a->N) * 2;
@@ -383,18 +391,24 @@ bool sf_linear_pp_ok(const sf_linear_args* a) {
   if ((a->residual && meets_y(a, a->residual, a->M, a->r_rs)) || (a->mul && meets_y(a, a->mul, a->mul_rows, a->mul_rs))) return false;
   // One round of 256 tiles here takes as long as about 540 of linear64_kernel's 128 x 128 tiles
   // (5120 x 3072 x 768: one round 33 us, 960 tiles 38; 3700 x 3072 x 768: one round 27 us, 696
-  // tiles 34; 5120 x 768 x 768: one round 24 us, 240 tiles 15)
-  const int64_t big = tiles(a, kTile);
-  return big < (1ll << 30) && 540 * ((big + 255) / 256) <= tiles(a, 128);
+  // tiles 34; 6000 x 1536 x 384: one round 19 us, 564 tiles 23; 5120 x 768 x 768: one round 24 us,
+  // 240 tiles 15), where this kernel's tiles cover at most half as much again as those.  Beyond that the
+  // two tie on some cards and it loses on others: 128 batched products of 300 x 304 x 320 (2 x 2 tiles
+  // against 3 x 3, 1.78 times the area) 28.0 here and 28.5 there on one card, 32.7 and 29.5 on another,
+  // 344 x 344 x 384 31.5 and 31.4, 37.3 and 32.7.  At 1.44 times the area 600 x 600 x 640 109 and 120, 110
+  // and 123 (520 x 520 x 576 85.4 and 85.2, 94.7 and 90.0); at 1.33 65536 x 264 x 768 56 and 67.
+  const int64_t big = tiles(a, kTile), small = tiles(a, 128), wgs = workgroups(a);
+  return big < (1ll << 30) && 540 * wgs * ((big + wgs - 1) / wgs) <= 256 * small && 8 * big <= 3 * small;
+}
+
+extern "C" int sf_hip_linear_large_tiles(const sf_linear_args* a) {
+  return a != nullptr && a->K % 64 == 0 && sf_linear_pp_ok(a);
 }
 
 int sf_linear_pp_launch(const sf_linear_args* a, hipStream_t stream) {
   const int64_t gx = (a->M + kTile - 1) / kTile, gy = ((int64_t)a->N + kTile - 1) / kTile;
   const int64_t total = tiles(a, kTile);
-  const void* kernel = a->glu ? reinterpret_cast<const void*>(linear_pp_kernel<true>) : reinterpret_cast<const void*>(linear_pp_kernel<false>);
-  // a multiple of 8 workgroups (XCDs), no more than are resident at once
-  const int64_t resident = std::max(8, sf_resident_workgroups(kernel, 512) / 8 * 8);
-  const dim3 grid((unsigned)std::min<int64_t>(resident, (total + 7) / 8 * 8));
+  const dim3 grid((unsigned)std::min<int64_t>(workgroups(a), (total + 7) / 8 * 8));
   if (a->glu) hipLaunchKernelGGL(linear_pp_kernel<true>, grid, dim3(512), 0, stream, *a, (int)gx, (int)gy, (int)total);
   else hipLaunchKernelGGL(linear_pp_kernel<false>, grid, dim3(512), 0, stream, *a, (int)gx, (int)gy, (int)total);
   return sf_check_launch("linear_pp_kernel");

@@ -3,7 +3,7 @@
 CPU: its tile order, the LDS layout of a step (what the copies write against what the operand
 reads fetch) and the epilogue's private block, restated from the kernel.  GPU: parity with an fp32
 product at the edges of its tiles and of its K steps, every epilogue, and the calls that must stay
-on the general kernels (an update in place)."""
+on the general kernels (an update in place).  Which kernel a call takes is asked of the library."""
 import ctypes
 
 import numpy as np
@@ -63,6 +63,56 @@ def test_epilogue_block_is_a_permutation(rb):
   assert np.array_equal(np.sort(slot.ravel()), np.arange(32 * rb // 16) * 16)
 
 
+def _args(M, N, K, *, x=1 << 32, wt=2 << 32, y=3 << 32, batch=0, **over):
+  """Arguments for the route query; the addresses are never dereferenced."""
+  from sparsefold_amd import _lib
+  a = _lib.LinearArgs()
+  a.M, a.N, a.K, a.mul_rows, a.batch = M, N, K, 1, batch
+  a.x, a.x_rs, a.wt, a.y, a.y_rs = x, K, wt, y, N
+  if batch > 1:
+    a.x_bs, a.w_bs, a.y_bs = M * K, N * K, M * N
+  for key, value in over.items():
+    setattr(a, key, value)
+  return a
+
+
+def _large_tiles(a):
+  from sparsefold_amd import _lib
+  return bool(_lib.load().sf_hip_linear_large_tiles(ctypes.byref(a)))
+
+
+# (M, N, K) of the parity cases: whole tiles; remainders of rows and columns (8 the smallest); the fewest K
+# steps; several tiles to a workgroup, the last round partly filled
+SHAPES = [(5120, 3072, 768), (3850, 3080, 192), (5000, 4104, 128), (6400, 6152, 448), (4097, 3576, 256)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_route_of_the_parity_shapes(M, N, K):
+  assert _large_tiles(_args(M, N, K))
+  assert _large_tiles(_args(M, N // 16 * 16, K, glu=1, y_rs=N // 16 * 8))
+  rows = 4 << 32
+  assert _large_tiles(_args(M, N, K, residual=rows, r_rs=N))
+  assert not _large_tiles(_args(M, N, K, y=rows, residual=rows, r_rs=N))       # in place
+  assert not _large_tiles(_args(M, N, K, y=rows, mul=rows + 2 * N * (M - 1), mul_rs=N))
+  # rows that are no whole number of 16-byte pieces, another output form, too few K steps
+  for over in ({"y": (3 << 32) + 2}, {"y_rs": N + 4}, {"yt": 5 << 32}, {"ycols": 8}, {"bias": (6 << 32) + 4}):
+    assert not _large_tiles(_args(M, N, K, **over)), over
+  assert not _large_tiles(_args(M, N, 64)) and not _large_tiles(_args(M, N, K + 8))
+
+
+@pytest.mark.parametrize("n,large", [(256, False), (257, False), (300, False), (344, False), (384, False),
+                                     (392, True), (436, True), (511, True), (600, True), (768, True), (1024, True)])
+def test_route_of_batched_products(n, large):
+  """128 planes of n x n: between one and one and a half tiles a side (257 .. 384) the smaller tiles win."""
+  assert _large_tiles(_args(n, (n + 7) // 8 * 8, (n + 63) // 64 * 64, batch=128)) == large
+
+
+@pytest.mark.parametrize("M,N,K,large", [(3700, 3072, 768, True), (6000, 1536, 384, True), (65536, 264, 768, True),
+                                         (5120, 768, 768, False), (1000, 3072, 768, False), (33000, 264, 768, False)])
+def test_route_of_single_products(M, N, K, large):
+  assert _large_tiles(_args(M, N, K)) == large
+
+
 def _check(y, ref, what):
   """bf16 rounding of the result (2^-8 of its value, half a step and the sum's fp32 error with it)."""
   err = (y.float() - ref).abs()
@@ -76,15 +126,14 @@ def _inputs(M, N, K, seed=3):
   return (r(M, K).bfloat16(), (r(N, K) / K ** 0.5).bfloat16(), r(N), r(M, N).bfloat16(), r(96, N).bfloat16())
 
 
-# whole tiles; remainders of rows and columns (8 the smallest); the fewest K steps; several tiles to
-# a workgroup, the last round partly filled
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(5120, 3072, 768), (3850, 3080, 192), (5000, 4104, 128), (6400, 6152, 448), (4097, 3576, 256)])
+@pytest.mark.parametrize("M,N,K", SHAPES)
 @pytest.mark.parametrize("epilogue", ["plain", "bias", "sigmoid_mul", "mul_residual", "glu"])
 def test_parity(M, N, K, epilogue):
   from sparsefold_amd import _lib
   from sparsefold_amd.backends.hip import ops
   x, w, b, res, mul = _inputs(M, N, K)
+  assert _large_tiles(_args(M, N, K))
   ref = x.float() @ w.float().t()
   if epilogue == "plain":
     _check(ops.linear(x, w), ref, epilogue)
@@ -103,6 +152,7 @@ def test_parity(M, N, K, epilogue):
     a.M, a.N, a.K, a.mul_rows, a.glu = M, n, K, 1, 1
     a.x, a.x_rs, a.wt = x.data_ptr(), K, w.data_ptr()
     a.y, a.y_rs = y.data_ptr(), n // 2
+    assert _large_tiles(a)
     _lib.check(_lib.load().sf_hip_linear_fwd(ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "linear")
     h = ref[:, :n]
     _check(y, torch.nn.functional.silu(h[:, 0::2]) * h[:, 1::2], epilogue)
@@ -117,7 +167,10 @@ def test_update_in_place_adds_its_residual_once():
   a = _lib.LinearArgs()
   a.M, a.N, a.K, a.mul_rows = M, N, K, 1
   a.x, a.x_rs, a.wt = x.data_ptr(), K, w.data_ptr()
-  a.y, a.y_rs, a.residual, a.r_rs = res.data_ptr(), N, res.data_ptr(), N
+  a.y, a.y_rs, a.residual, a.r_rs = torch.empty_like(res).data_ptr(), N, res.data_ptr(), N
+  assert _large_tiles(a)
+  a.y = res.data_ptr()
+  assert not _large_tiles(a)
   _lib.check(_lib.load().sf_hip_linear_fwd(ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "linear")
   _check(res, ref, "in place")
 
@@ -126,7 +179,8 @@ def test_update_in_place_adds_its_residual_once():
 @pytest.mark.parametrize("N", [300, 436, 511, 768])
 def test_products_of_the_triangle_multiplication(N):
   """The batched form (a plane per channel, several tiles to a workgroup), sizes whose rows are not a
-  whole number of pieces, against the 64-bit update."""
+  whole number of pieces, against the 64-bit update; 300 is the largest listed that takes smaller tiles."""
+  assert _large_tiles(_args(N, (N + 7) // 8 * 8, (N + 63) // 64 * 64, batch=128)) == (N > 384)
   from oracle import modules as OM
   from sparsefold_amd import workloads as W
   from sparsefold_amd import modules as M
