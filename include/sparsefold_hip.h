@@ -382,7 +382,8 @@ int sf_hip_cross_attention_fwd(const sf_cross_attention_args* a, void* workspace
  * x bf16 [S, N, C] (the condition [N, Cs] is shared by the S samples); w1 bf16 [2I, C] with
  * interleaved rows: row 2i = column i of the reference's [C, 2I] weight (the swish half), row
  * 2i + 1 = column I + i; w2 bf16 [C, I].  C % 64 == 0.  Workspace from
- * sf_hip_transition_workspace_bytes. */
+ * sf_hip_transition_workspace_bytes (0 where one kernel does it all: C = 128, I % 64 == 0 and no
+ * condition; the workspace may then be NULL). */
 typedef struct sf_transition_args {
   int32_t S, N, C, I, Cs;
   int32_t add_residual;

@@ -463,8 +463,9 @@ def transition_module(x: torch.Tensor, cond, w: dict, *, add_residual: bool = Tr
                "transition: precomputed conditioning must be bf16 [N, C] views with one row stride")
     a.pre_scale, a.pre_shift, a.pre_zgate, a.pre_rs = _vp(ps), _vp(pb), _vp(pz), rs
   lib = _lib.load()
-  ws = torch.empty(int(lib.sf_hip_transition_workspace_bytes(C.byref(a))), dtype=torch.uint8, device=x.device)
-  _lib.check(lib.sf_hip_transition_fwd(C.byref(a), _vp(ws), ws.numel(), _stream(x)), "sf_hip_transition_fwd")
+  nbytes = int(lib.sf_hip_transition_workspace_bytes(C.byref(a)))
+  ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device) if nbytes else None
+  _lib.check(lib.sf_hip_transition_fwd(C.byref(a), _vp(ws), nbytes, _stream(x)), "sf_hip_transition_fwd")
   return out.view(x.shape)
 
 

@@ -1059,6 +1059,7 @@ extern "C" int sf_hip_cross_attention_fwd(const sf_cross_attention_args* a, void
 namespace {
 
 size_t transition_ws(const sf_transition_args* a) {
+  if (sf_transition128_ok(a)) return 0;      // one kernel
   Arena ws{nullptr};
   const int64_t rows = (int64_t)a->S * a->N;
   const bool cond_gemms = a->cond && !a->pre_scale;
@@ -1096,12 +1097,12 @@ extern "C" int sf_hip_transition_fwd(const sf_transition_args* a, void* workspac
   if (!pre && a->cond && (a->w_scale == nullptr || a->w_shift == nullptr || a->w_zc == nullptr)) {
     sf_set_error("transition: a condition needs w_scale, w_shift and w_zc"); return 1;
   }
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (sf_transition128_ok(a)) return sf_transition128_launch(a, st);   // one kernel, no workspace
   if (workspace == nullptr || workspace_bytes < transition_ws(a)) {
     sf_set_error("transition: workspace of %zu bytes needed, %zu given", transition_ws(a), workspace_bytes);
     return 1;
   }
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (sf_transition128_ok(a)) return sf_transition128_launch(a, st);   // one kernel, no workspace
   Arena ws{static_cast<char*>(workspace)};
   const int64_t rows = (int64_t)a->S * a->N;
   int rc;

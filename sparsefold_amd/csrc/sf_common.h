@@ -151,8 +151,9 @@ int sf_attention_run(const sf_attention_args* a, void* workspace, size_t workspa
 // before it asks), and its launch.
 bool sf_linear_pp_ok(const sf_linear_args* a);
 int sf_linear_pp_launch(const sf_linear_args* a, hipStream_t stream);
-// Transition of 128 channels without a condition in one kernel: whether it serves `a` (sizes checked by
-// sf_hip_transition_fwd), and its launch.
+// Transition of 128 channels without a condition in one kernel, without a workspace: whether it serves
+// `a` (decided by the sizes; they are checked by sf_hip_transition_fwd), and its launch, which refuses
+// the addresses that the general path refuses.
 bool sf_transition128_ok(const sf_transition_args* a);
 int sf_transition128_launch(const sf_transition_args* a, hipStream_t stream);
 // Shared-bias attention (5 samples, head dim 48, one bias for every sample): whether it serves

@@ -30,6 +30,8 @@ constexpr int kP1 = kC + 8;            // LDS pitch (elements) of W1 rows and of
 constexpr int kP2 = 32 + 8;            // LDS pitch of W2 rows (32 intermediate channels)
 constexpr int kStage = 64 * kP1 + kC * kP2;   // elements of one weight stage
 
+typedef u32x4 u32x4_any __attribute__((aligned(2)));   // a 16-byte store at any even address (out alone may be one)
+
 struct TransArgs {
   int64_t rows; int I, items, add_residual;   // items = ceil(rows / 32)
   const uint16_t* x;                   // [rows, 128]
@@ -278,11 +280,11 @@ __global__ __launch_bounds__(64 * kWaves) void transition128_kernel(const TransA
     uint16_t* const op = a.out + (row0 + (lane >> 4)) * kC + 8 * (lane & 15);
     if (row0 + 32 <= a.rows) {
 #pragma unroll
-      for (int u = 0; u < 8; ++u) st16(op + 4 * u * kC, v[u]);
+      for (int u = 0; u < 8; ++u) *reinterpret_cast<u32x4_any*>(op + 4 * u * kC) = v[u];
     } else {
 #pragma unroll
       for (int u = 0; u < 8; ++u)
-        if (row0 + 4 * u + (lane >> 4) < a.rows) st16(op + 4 * u * kC, v[u]);
+        if (row0 + 4 * u + (lane >> 4) < a.rows) *reinterpret_cast<u32x4_any*>(op + 4 * u * kC) = v[u];
     }
     asm volatile("" ::: "memory");                       // (the rows are rewritten by the next item)
   }
@@ -292,12 +294,15 @@ bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 }  // namespace
 
+// By sizes alone: the workspace query must give the same answer whatever addresses the call comes with.
 bool sf_transition128_ok(const sf_transition_args* a) {
-  return a->C == kC && a->I % 64 == 0 && a->cond == nullptr && a->pre_scale == nullptr &&
-         (int64_t)a->S * a->N < (1ll << 35) && al16(a->x) && al16(a->out) && al16(a->w1) && al16(a->w2);
+  return a->C == kC && a->I % 64 == 0 && a->cond == nullptr && a->pre_scale == nullptr && (int64_t)a->S * a->N < (1ll << 35);
 }
 
 int sf_transition128_launch(const sf_transition_args* a, hipStream_t stream) {
+  if (!al16(a->x) || !al16(a->w1) || !al16(a->w2)) {
+    sf_set_error("transition: x, w1 and w2 must be 16-byte aligned"); return 1;
+  }
   TransArgs t{};
   t.rows = (int64_t)a->S * a->N; t.I = a->I; t.items = (int)((t.rows + 31) / 32); t.add_residual = a->add_residual;
   t.x = static_cast<const uint16_t*>(a->x); t.ln_w = a->ln_w; t.ln_b = a->ln_b;

@@ -66,6 +66,17 @@ def test_update_and_residual(rows, I, affine):
   _check(_call(x, torch.full_like(x, 7.0), ln_w, ln_b, w1, w2, True), x.double() + upd, upd, bound)
 
 
+@pytest.mark.parametrize("rows", [33, 300])
+def test_output_at_any_even_address_without_a_workspace(rows):
+  ln_w, ln_b, w1, w2, r = _weights(128, rows)
+  x = r(rows, 128).bfloat16()
+  want = _call(x, torch.empty_like(x), ln_w, ln_b, w1, w2, True)
+  buf = torch.full((rows * 128 + 8,), 7.0, device="cuda").bfloat16()
+  _call(x, buf[3:3 + rows * 128].view(rows, 128), ln_w, ln_b, w1, w2, True)
+  assert torch.equal(buf[3:3 + rows * 128].view(rows, 128), want)
+  assert bool((buf[:3] == 7).all()) and bool((buf[3 + rows * 128:] == 7).all())
+
+
 def test_in_place():
   ln_w, ln_b, w1, w2, r = _weights(512, 3)
   x = r(70001, 128).bfloat16()
