@@ -577,8 +577,8 @@ __device__ __forceinline__ void stage_out_weights(uint16_t* sW, uint16_t* sG, fl
   for (int n = tid; n < C; n += NTHR) sGoff[n] = goff[n];
 }
 
-// Gate block nb of 32 positions applied to the two o pieces of its chunks 2nb and 2nb + 1: D^T = W_g . X^T -> lane (position, half hf) holds gate row 8c + 4hf + e of the
-// block in register 4c + e.
+// Gate block nb of 32 positions applied to the two o pieces of its chunks 2nb and 2nb + 1:
+// D^T = W_g . X^T -> lane (position, half hf) holds gate row 8c + 4hf + e of the block in register 4c + e.
 //  KC = 2 (block = head nb): o operand chunk kk = 2nb + j of lane half h needs the gate of
 //    half j, register 8h + t -- one permlane32 swap per register pair gets it.
 //  KC = 1 (block = heads 2nb, 2nb + 1): chunk kk = 2nb + j of lane half h needs dims
@@ -991,7 +991,8 @@ __device__ __forceinline__ void tri_attn_body(const TriAttnArgs& a) {
     for (int k = 0; k < 4; ++k) breg[k] = ld16(p + 1024 * k);
   };
 
-  // Q operands (B of S^T = K Q^T) of a task's 4 rows.  Rows past N hold zeros and are never stored.
+  // Q operands (B of S^T = K Q^T) of a task's 4 rows.  q, k and v of rows past N are whatever the
+  // workspace held (the projection leaves them out); nothing of those rows is stored or flagged.
   bf16x8 qb8[kTR][KC];
   auto load_q = [&](int r0, int h, int qb, bf16x8 (&qd)[kTR][KC]) __attribute__((always_inline)) {
     const int iq = min(qb * 32 * kAW + 32 * wave + li, NP - 1);   // operand row (results of i >= N unused)
