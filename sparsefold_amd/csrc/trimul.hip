@@ -239,13 +239,13 @@ struct OutArgs {
   int N, Nt;                     // row length and stride (N rounded up to 8) of the product
   int64_t P, Pp;                 // N * Nt positions of a plane, and its stride
   const uint16_t* t;             // [128][Pp] channel-major product, rows of Nt
-  const uint16_t* z;             // [P, 128]
+  const uint16_t* z;             // [N * N, 128]
   const uint16_t* wo;            // folded output projection [128 out, 128 in]
   const float* oo;               // [128]
   const uint16_t* wg;            // folded gate [128 out, 128 in]
   const float* og;               // [128]
   int add_residual;
-  uint16_t* out;                 // [P, 128]
+  uint16_t* out;                 // [N * N, 128]
   int items, items_per_wave;     // blocks of 32 of the P positions
 };
 

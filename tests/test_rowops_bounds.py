@@ -2,7 +2,8 @@
 pair_logits128_kernel with 16-byte stores) and of the loads and stores of the window projection
 (csrc/modules.hip: adaln2_proj_kernel, one workgroup per side and worker), both of which store
 unconditionally: a lane whose plane, positions or row lie
-past the end stores the last valid plane's, chunk's or row's bytes again.  The host's tile
+past the end stores the last valid plane's, chunk's or row's bytes again.  Planes whose length is no
+multiple of 8 (one segment) end in 2-byte stores of the last P % 8 positions.  The host's tile
 arithmetic and the kernels' index expressions are restated; nothing here runs on a GPU.  Checked:
 every store lies inside the output, every output element is written, and a lane that repeats a
 store writes the element its owner writes (so the bytes are identical)."""
@@ -32,7 +33,7 @@ def test_pair_logits_every_tile_holds_a_plane():
 
 def _pl_stores(P, H, seg, grp, workers):
   """(element offset, plane, position) of every 16-byte store, and the element each lane's data
-  belongs to, for one launch with `workers` position workers."""
+  belongs to, and those of the tail's 2-byte stores, for one launch with `workers` position workers."""
   hb, g2, hgroups = _pl_tiles(H)
   NP, TPOS = 32 * hb, 32 * W
   LPP = TPOS // 8
@@ -40,7 +41,7 @@ def _pl_stores(P, H, seg, grp, workers):
   steps = (P + 31) // 32
   lane = np.arange(64)
   ch = lane % LPP
-  out = []
+  out, tail = [], []
   for worker in range(workers):
     for hg in range(hgroups):
       h0 = hg * g2 * NP
@@ -48,9 +49,20 @@ def _pl_stores(P, H, seg, grp, workers):
       while base < steps:
         for g in range(g2):
           p = base * 32 + 8 * ch
-          pc = np.minimum(p, P - 8)
+          pc = np.minimum(p, max((P & ~7) - 8, base * 32))
           chc = (pc - base * 32) >> 3
+          assert (chc >= 0).all() and (8 * chc + 7 < TPOS).all() and ((pc - base * 32) % 8 == 0).all()
           plmax = H - 1 - h0 - g * NP
+          if seg == P and P % 8 and base * 32 + TPOS >= P:        # the tail: one element per (plane, q)
+            t0, nt = (P & ~7) - base * 32, P & 7
+            assert 0 <= t0 and t0 + nt <= TPOS
+            e = np.arange(8 * NP)
+            pl, q = e >> 3, e & 7
+            keep = (q < nt) & (pl <= plmax)
+            hh = h0 + g * NP + pl[keep]
+            tail.append((hh * P + base * 32 + t0 + q[keep], hh, base * 32 + t0 + q[keep]))
+          if seg == P and base * 32 + 8 > P:                       # no whole chunk in the tile
+            continue
           for wave in range(W):
             for i in range(PPW // PPI):
               pl_own = wave * PPW + PPI * i + lane // LPP
@@ -62,7 +74,7 @@ def _pl_stores(P, H, seg, grp, workers):
               # the lane stores the tile row of plane pl, chunk chc: positions base*32 + 8 chc ..
               out.append((off, hh, base * 32 + 8 * chc))
         base += workers * W
-  return out
+  return out, tail
 
 
 @pytest.mark.parametrize("P,H,seg,grp", [(1320, 4, 1320, 4), (1320, 16, 1320, 16), (1320, 100, 1320, 100),
@@ -71,7 +83,8 @@ def _pl_stores(P, H, seg, grp, workers):
 @pytest.mark.parametrize("workers", [8, 16])
 def test_pair_logits_16_byte_stores(P, H, seg, grp, workers):
   assert P % 8 == 0 and seg % 8 == 0 and P % seg == 0 and H % grp == 0
-  stores = _pl_stores(P, H, seg, grp, workers)
+  stores, tail = _pl_stores(P, H, seg, grp, workers)
+  assert not tail
   total = H * P
   written = np.zeros(total, np.int64)
   for off, hh, p0 in stores:
@@ -84,6 +97,23 @@ def test_pair_logits_16_byte_stores(P, H, seg, grp, workers):
     assert (off == expect).all()
     for e in range(8):
       np.add.at(written, off + e, 1)
+  assert (written >= 1).all(), "every (plane, position) written"
+
+
+# from the shortest plane (8) over the ends of a chunk, of a tile (128) and of a step (32) to odd ones
+@pytest.mark.parametrize("P", [9, 15, 31, 33, 119, 121, 127, 129, 135, 259, 1023, 437 * 3])
+@pytest.mark.parametrize("H", [1, 16, 33, 64, 130])
+@pytest.mark.parametrize("workers", [8, 16])
+def test_pair_logits_planes_of_any_length(P, H, workers):
+  stores, tail = _pl_stores(P, H, P, H, workers)
+  written = np.zeros(H * P, np.int64)
+  for off, hh, p0 in stores:
+    assert (hh < H).all() and (p0 + 7 < P).all() and (off == hh * P + p0).all()
+    for e in range(8):
+      np.add.at(written, off + e, 1)
+  for off, hh, p in tail:
+    assert (hh < H).all() and (p < P).all() and (p >= P & ~7).all()
+    np.add.at(written, off, 1)
   assert (written >= 1).all(), "every (plane, position) written"
 
 

@@ -1,7 +1,8 @@
 """CPU model of the operand layouts and the global / LDS accesses of the dense triangle attention
-fast path (csrc/triangle.hip: tri_proj_kernel, tri_attn_kernel, tri_fixup_kernel and
-tri_out_kernel) for both of its instances -- KC = 2 (C = 128, head dim 32) and KC = 1 (C = 64,
-head dim 16) -- checked against the buffers the host carves, for N in {1, 37, 65, 257, 768}.
+fast path (csrc/triangle.hip: tri_fold_kernel's padding bias, tri_proj_kernel and its split form,
+tri_attn_kernel, tri_fixup_kernel, tri_out_kernel and its split form) for both of its instances --
+KC = 2 (C = 128, head dim 32) and KC = 1 (C = 64, head dim 16) -- checked against the buffers the host
+carves.
 The index expressions are the kernels' own, restated; nothing here runs on a GPU."""
 import numpy as np
 import pytest
@@ -116,8 +117,9 @@ def test_fast_path_accesses_stay_in_bounds(KC, N):
   # folded weight, offsets, flags and counters
   ws = int(_lib.load().sf_hip_triangle_workspace_bytes(N, C, H, D))
   assert ws >= 3 * 2 * E + 2 * EB + 2 * EO + (4 * C + 32) * C * 2
-  # projection: rows r < NP, positions p < NP; Q/K stores of head hd (16 bytes), V^T stores
-  r, p = NP - 1, NP - 1
+  # projection: rows r < N, positions p < NP; Q/K stores of head hd (16 bytes), V^T stores (the
+  # attention kernel reads the rows up to NP: below)
+  r, p = N - 1, NP - 1
   for hd in range(H):
     for kk in range(KC):
       assert _ql_off(KC, r, hd, NP, p, kk, 1) + 8 <= E
@@ -161,3 +163,115 @@ def test_fast_path_accesses_stay_in_bounds(KC, N):
           chunks.add(c16)
           assert _vl_off(KC, N - 1, H - 1, NP, c16, u & 1, D - 1) + 8 <= E
   assert chunks == set(range(NP // 16))
+
+
+# ---- the bias of the padding: filled by the fold kernel, the rest written by the projection ----
+
+def _fill(N, NP, transpose):
+  """fill_padding_bias: (query, key) and value (-1: -inf, 0) of every element of one head's pieces."""
+  q0, pc0 = (0, (N >> 6) * 8) if transpose else (N, 0)
+  pcs = NP // 8 - pc0
+  f = np.arange((NP - q0) * pcs)
+  js, i = 8 * (pc0 + f % pcs), q0 + f // pcs
+  e = np.arange(8)
+  s0 = (js[:, None] & 63) + e
+  j = (js[:, None] & ~63) + (s0 & 32) + 8 * ((s0 >> 2) & 3) + 4 * ((s0 >> 4) & 1) + (s0 & 3)
+  assert (_bias_pos64(j & 63) == s0).all()               # the stored position inverted
+  return np.broadcast_to(i[:, None], j.shape), j, np.where(j >= N, -1, 0)
+
+
+@pytest.mark.parametrize("transpose", [False, True])
+@pytest.mark.parametrize("N", [1, 31, 32, 37, 63, 64, 65, 96, 127, 128, 129, 192, 200, 257])
+def test_fill_and_projection_cover_the_bias(N, transpose):
+  """-inf for keys past N, 0 for the valid keys of queries past N, the projection's values (and the
+  masked logit) elsewhere: every element written, in that order of kernels, and none outside."""
+  NP = _np(N)
+  unset, pad, zero, value = 0, 1, 2, 3
+  state = np.full((NP, NP), unset)                       # [query][key]
+  if N != NP:
+    i, j, v = _fill(N, NP, transpose)
+    assert i.min() >= 0 and i.max() < NP and j.min() >= 0 and j.max() < NP
+    state[i, j] = np.where(v == -1, pad, zero)
+  # items of 32 positions p of rows r < N: query r, key p (starting node) or query p, key r
+  r, p = np.meshgrid(np.arange(N), np.arange(NP), indexing="ij")
+  za, zb = (p, r) if transpose else (r, p)
+  state[za, zb] = np.where(zb >= N, pad, np.where(za >= N, zero, value))
+  i, j = np.meshgrid(np.arange(NP), np.arange(NP), indexing="ij")
+  assert np.array_equal(state, np.where(j >= N, pad, np.where(i >= N, zero, value)))
+  # and the offsets of a head are a permutation of its plane
+  off = np.array([_bias_off(1, a, b, NP) for a, b in ((0, 0), (NP - 1, NP - 1))])
+  assert (off >= NP * NP).all() and (off < 2 * NP * NP).all()
+
+
+@pytest.mark.parametrize("NP", [128, 256])
+def test_bias_offsets_are_a_permutation(NP):
+  i, j = np.meshgrid(np.arange(NP), np.arange(NP), indexing="ij")
+  off = np.concatenate([_bias_off(h, i, j, NP).ravel() for h in range(2)])
+  assert np.array_equal(np.sort(off), np.arange(2 * NP * NP))
+
+
+# ---- the split projection and output stages (up to 512 items) ----
+
+@pytest.mark.parametrize("N", [1, 2, 31, 33, 64, 65, 100, 127, 128])
+def test_split_projection_takes_every_item_once(N):
+  """Grid (items / 4, 4 parts), a wave per item, no test for the end: the items are a multiple of 4."""
+  NP = _np(N)
+  items, bpr = N * (NP // 32), NP // 32
+  assert items <= 512 and items % 4 == 0
+  item = (np.arange(items // 4)[:, None] * 4 + np.arange(4)).ravel()
+  r, p0 = item // bpr, (item % bpr) * 32
+  assert r.max() < N and p0.max() + 32 <= NP
+  assert np.unique(r * NP + p0).size == items
+  for transpose in (False, True):
+    p = p0[:, None] + np.arange(32)
+    za, zb = (p, r[:, None]) if transpose else (r[:, None], p)
+    valid = (za < N) & (zb < N)
+    assert int(np.where(valid, za * N + zb, 0).max()) < N * N      # z and, by zb, the mask
+
+
+@pytest.mark.parametrize("KC", [1, 2])
+def test_split_projection_staging(KC):
+  """Part y's folded rows (q, k, v: C rows; bias: 32, the last repeated) and their place in LDS."""
+  C, cols = 64 * KC, (4 * 2 * KC + 1) * 32
+  stage = C * (C // 8) // 256
+  t = np.arange(256)[:, None] + 256 * np.arange(stage)[None, :]
+  for part in range(4):
+    rows, src = (32, 4 * C) if part == 3 else (C, C * part)
+    n = np.minimum(t // (C // 8), rows - 1)
+    assert (src + n).max() < cols and ((src + n) * C + (t % (C // 8)) * 8 + 7).max() < cols * C
+    assert rows <= 256 and src + rows <= cols
+  assert np.array_equal(np.unique(t // (C // 8)), np.arange(C))    # every LDS row is stored
+  assert (C - 1) * (C + 8) + C <= C * (C + 8)
+
+
+@pytest.mark.parametrize("KC", [1, 2])
+@pytest.mark.parametrize("N", [1, 31, 32, 33, 100, 127, 128])
+def test_split_output_writes_every_position_once(KC, N):
+  NB, C, NP = 2 * KC, 64 * KC, _np(N)
+  ib = (N + 31) >> 5
+  items = N * ib
+  assert items <= 512
+  lane = np.arange(64)
+  count = np.zeros((N, N, C // 8), np.int64)
+  for b in range(items):
+    r, i0 = b // ib, (b % ib) * 32
+    li = lane & 31
+    i = np.where(i0 + li < N, i0 + li, 0)                          # lanes past N read query 0
+    for wave in range(NB):
+      for j in range(2):                                           # o pieces 2 wave + j of the item
+        hd, hf, kk = _piece(KC, 2 * wave + j, lane >> 5)
+        assert (_o_off(KC, hd, r, i, hf, kk, N, NP) + 8 <= H * N * NP * 16 * KC).all()
+      for u in range(2):
+        row, ch = 16 * u + (lane >> 2), (lane & 3) * 8
+        keep = i0 + row < N
+        np.add.at(count, (np.full(64, r)[keep], (i0 + row)[keep], (32 * wave + ch)[keep] // 8), 1)
+  assert (count == 1).all()
+  # the waves' output rows (pitch 36) lie where W_g was, the gated o operands hold NC x 64 lanes x 8
+  assert NB * 32 * 36 <= C * (C + 8) and (2 * (NB - 1) + 1) * 64 * 8 + 63 * 8 + 8 <= (C // 16) * 64 * 8
+
+
+def _piece(KC, chunk, half):
+  """Head, piece and k-chunk of the output operand's 16-feature chunk for lane half `half`."""
+  if KC == 2:
+    return chunk >> 1, chunk & 1, half
+  return chunk, half, 0

@@ -1,24 +1,35 @@
 """CPU model of every global memory access of the triangle multiplicative update's kernels
 (csrc/trimul.hip: the prologue, the batched NT product through the library's GEMM, the epilogue)
-and of the host's launch arithmetic, checked against the buffer sizes the host allocates, for
-N in {1, 37, 64, 97, 384, 768} and both edges (97: N^2 = 9409 is not a multiple of the
-32-position block, so the last block of the epilogue has lanes past the end).  The index expressions are the kernels' own, restated;
-nothing here runs on a GPU."""
+and of the host's launch arithmetic, checked against the buffer sizes the host allocates, for both
+edges and sizes on both sides of each choice: the split prologue and epilogue (up to 512 items of 32
+positions, in 8 or 4 parts) and the persistent ones, linear64_kernel and linear_pp_kernel, rows of the
+product padded to 8 columns (N = 1, 37, 97, 129, 300, 437) and not, a last block of 32 positions that
+is partly past the end.  The index expressions are the kernels' own, restated; nothing here runs on a
+GPU."""
+import ctypes
+
 import numpy as np
 import pytest
 
 from sparsefold_amd import _lib
 
-KC, KTW = 128, 8                 # channels, waves per workgroup of the position kernels
+KC, KTW = 128, 8                 # channels, waves per workgroup of the persistent position kernels
+KWS, KTP, KOP = 136, 34, 36      # LDS pitches: weight rows, the staged product block, split output rows
 RESIDENT = 256                   # resident workgroups of the position kernels (one per CU)
+SPLIT_ITEMS, SPLIT_WAVES = 512, 4
+SIZES = [1, 37, 64, 97, 128, 129, 300, 437, 768]
 
 
 def _pn(n):
   return (n + 63) & ~63
 
 
+def _cols(n):
+  return (n + 7) & ~7
+
+
 def _pp(n):
-  return (n * n + 31) & ~31
+  return (n * _cols(n) + 31) & ~31
 
 
 def _grid(items):
@@ -32,125 +43,166 @@ def _grid(items):
 def _covered(items, ipw, groups):
   """Every item is processed by exactly one wave: workgroup g's wave w takes items
   g * KTW * ipw + k * KTW + w, k < ipw, until the first one past the end."""
-  seen = np.zeros(items, np.int64)
-  for g in range(groups):
-    for w in range(KTW):
-      for k in range(ipw):
-        item = g * KTW * ipw + k * KTW + w
-        if item >= items:
-          break
-        seen[item] += 1
-  return bool((seen == 1).all())
+  g, w, k = np.meshgrid(np.arange(groups), np.arange(KTW), np.arange(ipw), indexing="ij")
+  item = (g * KTW * ipw + k * KTW + w).ravel()
+  return np.array_equal(np.sort(item[item < items]), np.arange(items))
 
 
-def _proj_accesses(N, incoming):
-  Pn = _pn(N)
-  items = Pn * (Pn // 32)
-  ipw, groups = _grid(items)
-  assert _covered(items, ipw, groups)
-  item = np.arange(items)[:, None]
-  lane = np.arange(64)[None, :]
-  half, li = lane >> 5, lane & 31
-  cbs = Pn // 32
-  R, cb = item // cbs, item % cbs
-  col = 32 * cb + li
-  za, zb = (col, R) if incoming else (R, col)
-  ok = (za < N) & (zb < N)
-  # z reads, every lane (unconditional): 8 x 16 bytes at element (za * N + zb) * 128 + 8 * half
-  # + 16 kk, position 0 where not ok
-  zfirst = np.where(ok, za * N + zb, 0) * KC + 8 * half
-  zlast = zfirst + 16 * 7 + 7
-  z_max = int(zlast.max())
-  # mask reads, every lane: mask[za], mask[zb] where ok, mask[0] otherwise
-  m_max = int(np.where(ok, np.maximum(za, zb), 0).max())
-  # plane stores (2 bytes): lane (half, li) writes column col = 32 cb + li of plane row R for the
-  # channels 32 nb + 8 (r / 4) + 4 half + r % 4, r = 0..15, nb = 0..3
-  plane = Pn * Pn
-  pbase = R * Pn + col
-  # the kernel's byte address: uniform base dst + (32 nb + 8 (r / 4) + r % 4) plane * 2 plus the
-  # 64-bit lane offset (4 half plane + pbase) * 2 -- the same element as below
-  lofs = (4 * half * plane + pbase) * 2
-  assert (lofs % 2 == 0).all() and (lofs >= 0).all()
-  ch = np.array([[32 * nb + 8 * (r >> 2) + 4 * h + (r & 3) for nb in range(4) for r in range(16)] for h in (0, 1)])
-  chl = ch[half[0]]                                        # [64 lanes, 64 channels]
-  lo = int((chl.min(axis=1)[None, :] * plane + pbase).min())
-  hi = int((chl.max(axis=1)[None, :] * plane + pbase).max())
-  # every (channel, plane element) written exactly once
-  writes = np.zeros((KC, Pn * Pn), np.int64)
-  for h in (0, 1):
-    lanes = np.flatnonzero(half[0] == h)
-    for c in ch[h]:
-      np.add.at(writes[c], pbase[:, lanes].ravel(), 1)
-  return dict(items=items, z_max=z_max, m_max=m_max, plane_min=lo, plane_max=hi,
-              plane_elems=KC * plane, row_writes=writes, aligned8=True)
-
-
-def _gemm_accesses(N):
-  """linear64_kernel, batched: loads clamp rows to M-1 / N-1 and read k0 + swizzled piece < K
-  from rows of stride x_rs = K = Pn; stores y[b * y_bs + m * y_rs + n] for m < M, n < N."""
-  Pn = _pn(N)
-  M = Ng = N
-  K = Pn
-  x_rs, x_bs, y_rs, y_bs = Pn, Pn * Pn, N, _pp(N)
-  out = {}
-  for bm, bn in ((128, 128), (64, 128), (64, 64)):
-    gm, gn = (M + bm - 1) // bm, (Ng + bn - 1) // bn
-    # load rows: min(m0 + c * 8 + lane / 8, M - 1); columns k0 + rsw + 0..7 with k0 + 64 <= K
-    max_row = M - 1
-    max_col = K - 1                          # k0 <= K - 64, rsw + 7 <= 63
-    x_max = (KC - 1) * x_bs + max_row * x_rs + max_col
-    w_max = (KC - 1) * x_bs + (Ng - 1) * K + max_col
-    y_max = (KC - 1) * y_bs + (M - 1) * y_rs + (Ng - 1)
-    out[(bm, bn)] = (gm, gn, x_max, w_max, y_max)
-  return out, KC * Pn * Pn, KC * y_bs
-
-
-def _out_accesses(N):
-  P, Pp = N * N, _pp(N)
-  items = (P + 31) // 32
-  ipw, groups = _grid(items)
-  assert _covered(items, ipw, groups)
-  item = np.arange(items)[:, None]
-  lane = np.arange(64)[None, :]
-  half, li = lane >> 5, lane & 31
-  p = item * 32 + li
-  ok = p < P
-  qt = lane + 64 * np.arange(8)[:, None, None]            # the product loads: u = 0..7, every item
-  ct, seg = qt >> 2, qt & 3
-  t_start = ct * Pp + item[None] * 32 + 8 * seg
-  assert (t_start % 8 == 0).all(), "16-byte product loads aligned"
-  t_max = int((t_start + 7).max())
-  # the wave's LDS rows hold 32 x kWS (136) elements; the staged block sits at pitch 34
-  lds_store = (ct * 34 + 8 * seg + 7).max()
-  kk, e = np.arange(8)[:, None, None, None], np.arange(4)[None, :, None, None]
-  lds_read = ((16 * kk + 8 * half[None] + 2 * e + 1) * 34 + li[None]).max()
-  assert max(lds_store, lds_read) < 32 * 136 and ((ct * 34 + 8 * seg) % 2 == 0).all()
-  z_max = int((p * KC + 8 * half + 16 * 7 + 7)[ok].max())
-  q = lane + 64 * np.arange(8)[:, None, None]             # the row-store loop: u = 0..7
-  pos, c8 = q >> 4, (q & 15) * 8
-  pp = item[None] * 32 + pos
-  okw = pp < P
-  out_max = int((pp * KC + c8 + 7)[okw].max())
-  return dict(t_max=t_max, t_elems=KC * Pp, z_max=z_max, out_max=out_max, elems=P * KC)
+def _proj_parts(items):
+  """(first channel row of the parts, blocks of 32 channels in each): blockIdx.y of the split kernel,
+  or all 8 blocks in turn."""
+  if items > SPLIT_ITEMS:
+    return [0], 8
+  bpw = 1 if items <= 128 else 2
+  return [32 * bpw * y for y in range(8 // bpw)], bpw
 
 
 @pytest.mark.parametrize("incoming", [False, True])
-@pytest.mark.parametrize("N", [1, 37, 64, 97, 384, 768])
-def test_trimul_kernel_accesses_stay_in_bounds(N, incoming):
-  pr = _proj_accesses(N, incoming)
-  assert pr["z_max"] < N * N * KC and pr["m_max"] < N
-  assert 0 <= pr["plane_min"] and pr["plane_max"] < pr["plane_elems"]
-  assert pr["aligned8"]
-  assert (pr["row_writes"] == 1).all(), "every channel's padded plane element written exactly once (zeros included)"
-  gemm, ab_elems, t_elems = _gemm_accesses(N)
-  for (bm, bn), (gm, gn, x_max, w_max, y_max) in gemm.items():
-    assert x_max < ab_elems and w_max < ab_elems and y_max < t_elems, (bm, bn)
-    assert gm * gn * KC > 0 and gm < 2 ** 31 and KC <= 65535
-  o = _out_accesses(N)
-  assert o["t_max"] < o["t_elems"] and o["z_max"] < o["elems"] and o["out_max"] < o["elems"]
+@pytest.mark.parametrize("N", SIZES)
+def test_prologue(N, incoming):
+  Pn = _pn(N)
+  items, cbs = Pn * (Pn // 32), Pn // 32
+  if items > SPLIT_ITEMS:
+    assert _covered(items, *_grid(items))
+  else:
+    assert items % SPLIT_WAVES == 0              # item = 4 blockIdx.x + wave, no test for the end
+  item = np.arange(items)[:, None]
+  lane = np.arange(64)[None, :]
+  half, li = lane >> 5, lane & 31
+  R, col = item // cbs, 32 * (item % cbs) + li
+  za, zb = (col, R) if incoming else (R, col)
+  ok = (za < N) & (zb < N)
+  # z reads, every lane (unconditional): 8 x 16 bytes at element (za * N + zb) * 128 + 8 * half
+  # + 16 kk, position 0 where not ok; mask[za], mask[zb] likewise
+  assert int((np.where(ok, za * N + zb, 0) * KC + 8 * half).max()) + 16 * 7 + 7 < N * N * KC
+  assert int(np.where(ok, np.maximum(za, zb), 0).max()) < N
+  # plane stores (2 bytes): the uniform base of channel 32 nb + 8 (r / 4) + r % 4 plus the lane offset
+  # (4 half plane + R Pn + col): every element of both sides' 128 planes exactly once
+  plane = Pn * Pn
+  pos = R * Pn + col
+  rows, bpw = _proj_parts(items)
+  seen = np.zeros(2 * KC, np.int64)              # (side, channel) rows taken by the parts
+  lanes = [pos[:, np.flatnonzero(half[0] == h)].ravel() for h in (0, 1)]
+  for h in (0, 1):
+    assert np.array_equal(np.sort(lanes[h]), np.arange(plane))    # a half's lanes cover a plane once
+  for rg in rows:
+    for j in range(bpw):
+      first = rg + 32 * j                        # gate row of the block: side kC + channel
+      side, ch0 = first // KC, first % KC
+      assert (rg % KC) + 32 * j < KC or bpw == 8
+      for h in (0, 1):
+        for r in range(16):
+          ch = ch0 + 8 * (r >> 2) + 4 * h + (r & 3)
+          seen[side * KC + ch] += 1
+          assert 0 <= ch * plane + int(lanes[h].min()) and ch * plane + int(lanes[h].max()) < KC * plane
+  assert (seen == 1).all()
 
 
-@pytest.mark.parametrize("N", [1, 37, 64, 384, 768])
+@pytest.mark.parametrize("bpw", [1, 2])
+def test_split_prologue_staging(bpw):
+  """The part's gate and projection rows: every LDS row from its own weight row, no access past either."""
+  G = 32 * bpw
+  stage = 2 * G * (KC // 8) // 256
+  t = np.arange(256)[:, None] + 256 * np.arange(stage)[None, :]
+  n, c8 = t >> 4, (t & 15) * 8
+  assert np.array_equal(np.unique(n * KC + c8), np.arange(2 * G * KC // 8) * 8)
+  for y in range(8 // bpw):
+    rg = G * y
+    row = (n // G) * 2 * KC + rg + n % G
+    assert row.max() < 4 * KC                                       # folded GLU rows
+    # LDS row j of the gate half is channel row rg + j, of the projection half 2 kC + rg + j
+    assert all(((row == rg + j) == (n == j)).all() and ((row == 2 * KC + rg + j) == (n == G + j)).all() for j in (0, G - 1))
+    tid = np.arange(2 * G)
+    assert ((tid // G) * 2 * KC + rg + tid % G).max() < 4 * KC
+  assert 2 * G <= 256 and (2 * G - 1) * KWS + KC <= bpw * 64 * KWS
+
+
+def _large_tiles(N):
+  a = _lib.LinearArgs()
+  a.M, a.N, a.K, a.mul_rows, a.batch = N, _cols(N), _pn(N), 1, KC
+  a.x, a.wt, a.y = 1 << 32, 2 << 32, 3 << 32
+  a.x_rs, a.y_rs, a.x_bs, a.w_bs, a.y_bs = _pn(N), _cols(N), _pn(N) ** 2, _pn(N) ** 2, _pp(N)
+  return bool(_lib.load().sf_hip_linear_large_tiles(ctypes.byref(a)))
+
+
+@pytest.mark.parametrize("N", SIZES)
+def test_product(N):
+  """Loads clamp rows to M - 1 / N - 1 of the planes (rows of K = Pn); the product's rows hold Nt
+  columns, all of them stored."""
+  Pn, Nt = _pn(N), _cols(N)
+  assert Nt <= Pn and Pn % 64 == 0                     # the columns past N come from planes' zero rows
+  ab, t_elems = KC * Pn * Pn, KC * _pp(N)
+  assert (KC - 1) * Pn * Pn + (N - 1) * Pn + Pn - 1 < ab and (KC - 1) * Pn * Pn + (Nt - 1) * Pn + Pn - 1 < ab
+  assert (KC - 1) * _pp(N) + (N - 1) * Nt + Nt - 1 < t_elems
+  written = np.zeros((N, Nt), np.int64)
+  if _large_tiles(N):
+    assert N > 384
+    # a wave's part: 128 rows x 64 columns in blocks of 32 rows; lane: row 8 i + lane / 8, piece lane % 8,
+    # rows past the end the last row, pieces past the end the last valid one (the same bytes again)
+    lane = np.arange(64)
+    for bx in range((N + 255) // 256):
+      for by in range((Nt + 255) // 256):
+        for wave in range(8):
+          m0, n0 = 256 * bx + 128 * (wave // 4), 256 * by + 64 * (wave % 4)
+          if n0 >= Nt:
+            continue
+          pc = np.minimum(lane % 8, (Nt - n0) // 8 - 1)
+          for mb in range(4):
+            for i in range(4):
+              m = np.minimum(m0 + 32 * mb + 8 * i + lane // 8, N - 1)
+              assert (n0 + 8 * pc + 7 < Nt).all() and ((m * Nt + n0 + 8 * pc) % 8 == 0).all()
+              for e in range(8):
+                np.add.at(written, (m, n0 + 8 * pc + e), 1)
+    assert (written >= 1).all()
+  else:
+    for bm, bn in ((128, 128), (64, 128), (64, 64)):
+      gm, gn = (N + bm - 1) // bm, (Nt + bn - 1) // bn
+      assert gm * bm >= N and gn * bn >= Nt and gm < 2 ** 31 and KC <= 65535
+
+
+def _positions(N, items):
+  """out_position of the 32 positions of every item: the element of z and out, or -1."""
+  p = np.arange(items * 32).reshape(items, 32)
+  row, col = p // _cols(N), p % _cols(N)
+  return np.where((p < N * _cols(N)) & (col < N), row * N + col, -1)
+
+
+@pytest.mark.parametrize("N", SIZES)
+def test_epilogue(N):
+  Pp = _pp(N)
+  items = (N * _cols(N) + 31) // 32
+  split = items <= SPLIT_ITEMS
+  if not split:
+    assert _covered(items, *_grid(items))
+  pos = _positions(N, items)
+  assert np.array_equal(np.sort(pos[pos >= 0]), np.arange(N * N))   # every position of z and out once
+  # the product loads, 16 bytes each, whatever the position: channel w / 4, pieces of 8 positions
+  threads, loads = (256, 2) if split else (64, 8)
+  w = np.arange(threads)[:, None] + threads * np.arange(loads)[None, :]
+  c, seg = w >> 2, w & 3
+  start = c * Pp + (items - 1) * 32 + 8 * seg
+  assert (start % 8 == 0).all() and int(start.max()) + 7 < KC * Pp
+  assert np.array_equal(np.sort((c * 32 + 8 * seg).ravel()), np.arange(KC * 32 // 8) * 8)
+  # staged at pitch 34 and read back as channels 16 kk + 8 half + 0..7 of position li
+  lds = 4 * 32 * KOP if split else 32 * KWS
+  assert int((c * KTP + 8 * seg + 7).max()) < lds and ((c * KTP + 8 * seg) % 2 == 0).all()
+  assert (16 * 7 + 8 + 2 * 3 + 1) * KTP + 31 < lds
+  # z: every lane, position 0 where there is none
+  assert int(np.maximum(pos, 0).max()) * KC + 8 + 16 * 7 + 7 < N * N * KC
+  if split:
+    # residual and output of wave w: channels 32 w + 8 g + 4 half .. + 3, and whole pieces of 8 through LDS
+    lane = np.arange(64)
+    got = sorted((16 * u + l // 4, 32 * wv + (l % 4) * 8) for wv in range(4) for u in range(2) for l in lane)
+    assert got == [(r, 8 * k) for r in range(32) for k in range(16)]
+    assert 3 * 32 * KOP + 31 * KOP + 24 + 7 < lds
+    assert 32 * 3 + 8 * 3 + 4 + 3 < KC
+  else:
+    w = np.arange(64)[:, None] + 64 * np.arange(8)[None, :]
+    got = sorted(zip((w >> 4).ravel().tolist(), ((w & 15) * 8).ravel().tolist()))
+    assert got == [(r, 8 * k) for r in range(32) for k in range(16)]
+
+
+@pytest.mark.parametrize("N", SIZES)
 def test_trimul_workspace_covers_the_modelled_buffers(N):
   lib = _lib.load()
   Pn, Pp = _pn(N), _pp(N)
