@@ -1,7 +1,8 @@
 """The 256 x 256-tile GEMM behind sf_hip_linear_fwd (csrc/linear_pp.hip).
 
-CPU: its tile order, the LDS layout of a step (what the copies write against what the operand
-reads fetch) and the epilogue's private block, restated from the kernel.  GPU: parity with an fp32
+CPU: its tile order, the addresses of its copies and stores at the operands' edges, the LDS layout of a
+step (what the copies write against what the operand reads fetch) and the epilogue's private block,
+restated from the kernel.  GPU: parity with an fp32
 product at the edges of its tiles and of its K steps, every epilogue, and the calls that must stay
 on the general kernels (an update in place).  Which kernel a call takes is asked of the library."""
 import ctypes
@@ -54,6 +55,56 @@ def test_step_layout_and_bank_groups():
         assert addr[l] == where[(32 * block + li[l], 2 * kk + half[l])]
       for g in range(4):
         assert np.unique(addr[16 * g:16 * g + 16] % 256).size == 16
+
+
+@pytest.mark.parametrize("M,N,K,pad", [(256, 256, 128, 0), (3850, 3080, 192, 0), (300, 272, 128, 8), (4097, 3576, 256, 64), (257, 8, 320, 0)])
+def test_copies_stay_inside_the_operands(M, N, K, pad):
+  """Every 16-byte piece a step's copies read, at the tiles on the operands' edges: rows past the end
+  read the last row, 32-bit lane offsets, x rows at a stride of K + pad."""
+  lane = np.arange(64)
+  crow, cpiece = lane >> 2, (lane & 3) ^ ((lane >> 4) & 3)
+  for rows, rs, waves in ((M, K + pad, range(4)), (N, K, range(4, 8))):
+    size = ((rows - 1) * rs + K) * 2
+    pieces = set()
+    for b in range((rows + TILE - 1) // TILE):
+      r0 = b * TILE
+      lastr = rows - 1 - r0
+      for wave in waves:
+        for u in range(4):
+          local = np.minimum(16 * ((wave % 4) * 4 + u) + crow, lastr)
+          vo = local * 2 * rs + cpiece * 16
+          assert (vo >= 0).all() and (vo < 1 << 32).all()
+          for t in range(K // 32):
+            at = r0 * rs * 2 + vo + t * 64
+            assert (at + 16 <= size).all()
+            pieces.update(zip((r0 + local).tolist(), (4 * t + cpiece).tolist()))
+    assert pieces == {(r, p) for r in range(rows) for p in range(K // 8)}     # every piece of every row
+
+
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("M,N", [(256, 256), (300, 272), (129, 16), (511, 1040), (257, 528)])
+def test_stores_cover_the_result(M, N, glu):
+  """Rows past the end store the last row again, columns past the end the last valid piece, a wave with no
+  column nothing: inside the result, each lane the element its data belongs to, all of it."""
+  ncols, rb = (N // 2, 64) if glu else (N, 128)
+  rp = rb // 16
+  lane = np.arange(64)
+  written = np.zeros((M, ncols), np.int64)
+  for bx in range((M + TILE - 1) // TILE):
+    for by in range((N + TILE - 1) // TILE):
+      for wave in range(8):
+        m0, n0 = bx * TILE + 128 * (wave // 4), by * TILE + 64 * (wave % 4)
+        nc0 = n0 // 2 if glu else n0
+        if nc0 >= ncols:
+          continue
+        pc = np.minimum(lane % rp, (ncols - nc0) // 8 - 1)
+        for mb in range(4):
+          for i in range(32 // (64 // rp)):
+            m = np.minimum(m0 + 32 * mb + i * (64 // rp) + lane // rp, M - 1)
+            assert (pc >= 0).all() and (nc0 + 8 * pc + 7 < ncols).all()
+            for e in range(8):
+              np.add.at(written, (m, nc0 + 8 * pc + e), 1)
+  assert (written >= 1).all()
 
 
 @pytest.mark.parametrize("rb", [128, 64])
