@@ -2129,9 +2129,11 @@ float sum_limit(float requested) {
 
 // Items (of 32 positions) up to which the projection and the output stage run split: two waves per
 // SIMD of the unsplit kernels' 8-wave workgroups would then fill at most a quarter of the chip.
-// Whole call at C = 128, us, unsplit against split (the host takes 35 of it): projection N = 64
-// 37.7 / 35.9, 150 (2048 items) 47.5 / 59.4; output N = 64 37.7 / 34.2, 128 (512) 39.1 / 37.5,
-// 150 (750) 47.5 / 49.3, 200 (1400) 50.1 / 60.3.
+// GPU time of the whole call (graph replay), us, unsplit / split, with the stage's items.  C = 128,
+// projection: N = 20 29.5 / 23.6, 128 (512) 37.3 / 33.1, 129 (1032) 45.3 / 45.9, 200 (1600) 48.0 / 51.8;
+// output: N = 20 28.2 / 23.6, 128 (512) 34.9 / 33.1, 129 (645) 45.3 / 46.5, 200 (1400) 48.0 / 56.0.
+// C = 64, projection: N = 128 28.2 / 25.0, 129 33.4 / 33.2, 200 36.7 / 39.1; output: 24.8 / 25.0,
+// 33.2 / 33.4, 36.9 / 38.2.
 constexpr int kSplitItems = 512;
 
 template <int KC>

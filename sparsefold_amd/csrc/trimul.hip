@@ -508,9 +508,9 @@ size_t ws_bytes(int N) { return carve(nullptr, N).bytes; }
 
 // Items (of 32 positions) up to which the projection and the output stage run split: two waves per
 // SIMD of the unsplit kernels' 8-wave workgroups would then fill at most a quarter of the chip.
-// Whole call, us, unsplit against split: projection N = 64 36.4 / 27.7, 128 (512 items) 41.1 / 36.3,
-// 200 (2048) 52.2 / 62.1; output N = 64 36.4 / 30.6, 128 (512) 41.1 / 38.9, 150 (713) 49.0 / 49.0,
-// 200 (1250) 52.2 / 59.0.
+// GPU time of the whole call (graph replay), us, unsplit / split, with the stage's items.  Projection:
+// N = 20 27.9 / 18.6, 64 30.3 / 21.0, 128 (512) 39.3 / 33.0, 129 (1152) 49.3 / 47.5, 200 (2048) 50.4 / 52.8;
+// output: N = 20 24.7 / 18.6, 128 (512) 34.6 / 33.0, 129 (549) 49.4 / 49.8, 200 (1250) 50.5 / 56.1.
 constexpr int kSplitItems = 512;
 
 int launch_grid(const void* kernel, int items) {
