@@ -206,9 +206,9 @@ __global__ __launch_bounds__(256) void attention_fwd_kernel(const sf_attention_a
 //         16-byte pieces of a K row are XOR-swizzled by key so that the S^T operand reads of
 //         consecutive lanes hit distinct banks)
 //   S^T   = K Q^T
-//   P     = 2^(t - m) of the fp32 logits t = scale log2(e) S^T + log2(e) bias, with m near the row's
-//         maximum; masked keys have t = SF_MASKED_LOGIT and keys past K weigh 0; lane half h holds
-//         keys 8c + 4h + e of each 32-key half
+//   P     = e^(t - m) of the fp32 logits t = scale S^T + bias, with m near the row's maximum; masked
+//         keys have t = kMaskedLogit and keys past K weigh 0; lane half h holds keys 8c + 4h + e of
+//         each 32-key half
 //   O^T  += V^T P^T, the V^T operand read straight from the row-major V tile with
 //         ds_read_b64_tr_b16: lane (d, h) of 16-lane group G gets the 4 keys the matching P^T
 //         lane holds, for one dim -- no transposed copy of V is ever made.
@@ -221,7 +221,24 @@ typedef __attribute__((address_space(3))) uint32_t lds_u32a;
 typedef short v4i16 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
 
+constexpr float kMaskedLogit = SF_MASKED_LOGIT / SF_LOG2E;   // a masked key's logit, natural units
 constexpr float kMassLimit = 1.152921504606846976e18f;   // 2^60: weight mass of a tile that moves m
+
+// A reference point m of logits t (natural units): weights are 2^(t l2 - ml), one fma and one exp2.  l2 =
+// log2 e and ml = m l2 rounded: what the rounding lost scales every weight of the row alike.  From
+// 2^28 on it could overflow them (2^102 at 2e38), so there l2 = 1: logits of that size differ by 32 or
+// not at all, and e^-32 and 2^-32 both weigh nothing.
+struct Attn2Ref {
+  float l2, ml;
+  __device__ __forceinline__ explicit Attn2Ref(float m) : l2(fabsf(m) < 0x1p28f ? SF_LOG2E : 1.f), ml(m * l2) {
+    asm volatile("" : "+v"(ml));                             // (rounded once: not fused into what uses it)
+  }
+};
+// What sums against m are worth against mnew >= m.
+__device__ __forceinline__ float attn2_rescale(float m, float mnew) {
+  const Attn2Ref a(m), b(mnew);
+  return a.l2 == b.l2 ? fast_exp2(a.ml - b.ml) : 0.f;
+}
 
 struct Attn2Plan {
   int QB;            // 32-query blocks per (batch, head)
@@ -344,7 +361,7 @@ __global__ __launch_bounds__(256, SHARED && (DP == 32 || (KC <= 3 && BL < 2)) ? 
     const int d0 = 16 * kk + 8 * half;
     qb[kk] = as_bf16x8(d0 < D ? ld16(qp + (int64_t)iq * a.q_s[2] + d0) : u32x4{0, 0, 0, 0});
   }
-  const float cs = a.scale * SF_LOG2E;
+  const float scale = a.scale;
 
   // ---- tile copy: chunk c of a tile, K chunks first ----
   uint8_t* wsm = smem + (SHARED ? 0 : wave * 2 * T::kBufBytes);
@@ -510,11 +527,10 @@ __global__ __launch_bounds__(256, SHARED && (DP == 32 || (KC <= 3 && BL < 2)) ? 
       load_side(j0 + 64);
     }
     if (wactive) {
-      // ---- logits s = scale log2(e) (S^T = K Q^T) + log2(e) bias; register r of half kb is key
-      //      32 kb + 8 (r / 4) + 4 half + r % 4 of the tile.  A masked key's is SF_MASKED_LOGIT
-      //      whatever its q.k and bias are (NaN included), a key's past K is -inf; a masked query
-      //      masks every key.  They are rounded before m is subtracted: in one fma with -m, what the
-      //      rounding of a large m had lost (2^103 at a bias of 2e38) became the difference. ----
+      // ---- logits s = scale (S^T = K Q^T) + bias; register r of half kb is key
+      //      32 kb + 8 (r / 4) + 4 half + r % 4 of the tile.  A masked key's is kMaskedLogit whatever
+      //      its q.k and bias are (NaN included), a key's past K is -inf; a masked query masks every
+      //      key. ----
       f32x16 s[2];
       auto logits = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -535,7 +551,7 @@ __global__ __launch_bounds__(256, SHARED && (DP == 32 || (KC <= 3 && BL < 2)) ? 
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             const uint32_t w = bcur[4 * kb + (r >> 2)][(r >> 1) & 1];
-            s[kb][r] = __builtin_fmaf(s[kb][r], cs, ((r & 1) ? bfhi(w) : bflo(w)) * SF_LOG2E);
+            s[kb][r] = __builtin_fmaf(s[kb][r], scale, (r & 1) ? bfhi(w) : bflo(w));
           }
         }
         if (mbits != ~0ull || any_qmasked) {                 // uniform
@@ -554,11 +570,11 @@ __global__ __launch_bounds__(256, SHARED && (DP == 32 || (KC <= 3 && BL < 2)) ? 
             }
           };
           const uint64_t below = j0 + 64 <= K ? ~0ull : ~0ull >> (j0 + 64 - K);   // keys below K
-          if (mbits != below || any_qmasked) replace(mbits, qvalid, SF_MASKED_LOGIT);
+          if (mbits != below || any_qmasked) replace(mbits, qvalid, kMaskedLogit);
           if (below != ~0ull) replace(below, true, -INFINITY);
         }
       };
-      // ---- softmax against a reference point m (log2 units) ----
+      // ---- softmax against a reference point m ----
       // The first tile sets m to the row maximum of its 64 keys.  Later tiles keep it unless the
       // probability mass of the tile exceeds kMassLimit (all weights are >= 0, so the sum bounds
       // every weight and an overflow cannot pass unnoticed); then m moves to the tile's maximum
@@ -572,12 +588,6 @@ __global__ __launch_bounds__(256, SHARED && (DP == 32 || (KC <= 3 && BL < 2)) ? 
 #pragma unroll
           for (int r = 0; r < 16; ++r) v = fmaxf(v, s[kb][r]);
         return fmaxf(v, __shfl_xor(v, 32));
-      };
-      auto subtract = [&](float mref) __attribute__((always_inline)) {
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) s[kb][r] -= mref;
       };
       auto weights = [&](bf16x2 (&pw)[16]) __attribute__((always_inline)) {
         float t0 = 0.f, t1 = 0.f;
@@ -598,7 +608,7 @@ __global__ __launch_bounds__(256, SHARED && (DP == 32 || (KC <= 3 && BL < 2)) ? 
         logits();
         if (raise) {
           const float mnew = fmaxf(m, row_max());
-          const float alpha = fast_exp2(m - mnew);
+          const float alpha = attn2_rescale(m, mnew);
           m = mnew;
           l *= alpha;
 #pragma unroll
@@ -606,7 +616,11 @@ __global__ __launch_bounds__(256, SHARED && (DP == 32 || (KC <= 3 && BL < 2)) ? 
 #pragma unroll
             for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
         }
-        subtract(m);
+        const Attn2Ref ref(m);
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) s[kb][r] = __builtin_fmaf(s[kb][r], ref.l2, -ref.ml);
         ts = weights(pw);
         if (raise || !__any(!(ts <= kMassLimit))) break;
       }
@@ -697,7 +711,7 @@ __global__ __launch_bounds__(256, SHARED && (DP == 32 || (KC <= 3 && BL < 2)) ? 
 
 // Combine of the key-range slices: thread per (query block, query, 4 dims).  O and l of each
 // slice are relative to the slice's own reference point m_s; with M = max m_s the result is
-// sum_s O_s 2^(m_s - M) / sum_s l_s 2^(m_s - M), then the gate.  All loads of a thread
+// sum_s O_s w_s / sum_s l_s w_s, w_s = attn2_rescale(m_s, M), then the gate.  All loads of a thread
 // are independent and issued together: one memory round trip per thread.
 template <int DP, int KS>
 __global__ __launch_bounds__(256) void attn2_combine_kernel(const sf_attention_args a, const Attn2Plan pl) {
@@ -733,7 +747,7 @@ __global__ __launch_bounds__(256) void attn2_combine_kernel(const sf_attention_a
   float lsum = 0.f, v[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int sl = 0; sl < KS; ++sl) {
-    const float w = fast_exp2(ml[sl][0] - mx);
+    const float w = attn2_rescale(ml[sl][0], mx);
     lsum += w * ml[sl][1];
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] += w * os[sl][e];
