@@ -13,7 +13,9 @@
 // (W1) of channels 32 (i + 1) .. and the second (W2) of channels 32 i ..: the gating of one block of
 // channels sits in the shadow of the next block's MFMAs.
 //
-// 147456 rows (N = 384): 205 -> 80 us for the call.  A pass of 256 rows a workgroup takes 24 us: 11 us
+// 147456 rows (N = 384): 206 -> 75 us for the call, 5000 (N = 70) 34 -> 22: the host's part, one launch
+// for three.  (On the GPU a pass is 23 us however few rows there are, the three launches 15 to 18 up to
+// 4096: replayed from a graph, such calls took less before.)  A pass of 256 rows a workgroup takes 24 us: 11 us
 // of MFMAs (384 a wave, two waves per SIMD), 5 of gating beside them, 4 of LayerNorm, 2 of stores, the
 // rest operand reads, barriers and staging.  Built and not kept: the two waves of a SIMD changing
 // rows two steps apart (the barrier of every step makes one wait through the other's change: 26 us).

@@ -51,8 +51,10 @@ def test_minus_infinity_over_whole_tiles(Q, K, D, schedule):
   bias[1, :, 5:, 64:192] = -INF                        # tiles in between
   bias[1, 1, :5, :K - 1] = -INF                        # all but the last key
   _check(q, k, v, bias, mask, schedule)
-  bias[bias == -INF] = torch.finfo(torch.bfloat16).min # the other usual way to exclude keys
-  _check(q, k, v, bias, mask, schedule)
+  excluded = bias == -INF
+  for value in (torch.finfo(torch.bfloat16).min, -1e9):  # the other usual ways to exclude keys
+    bias[excluded] = value
+    _check(q, k, v, bias, mask, schedule)
 
 
 @pytest.mark.parametrize("D", [24, 48])
