@@ -26,9 +26,9 @@
 //
 // Measured against linear64_kernel (random bf16 data, us a call): 8192 x 8192 x 1024 134 against 174,
 // 5120 x 3072 x 768 32 against 38, 3700 x 3072 x 768 27 against 35, 128 batched 768^3 148 against 196
-// (the triangle multiplication around them 412 against 464).  What is left at 5120 x 3072 x 768: 7 us of
-// launch, first copies and barriers, 5 us of result stores at the memory's write rate, 18 us of
-// MFMAs at the clock the matrix cores hold on random data.
+// (the triangle multiplication around them 411 against 458).  At 5120 x 3072 x 768 (a tile for each of 240
+// workgroups) a workgroup is resident for 47 thousand cycles, and its SIMDs' matrix cores are busy for 24.6
+// of them; the rest is first copies, barriers and the result's stores (5 us at the memory's write rate).
 #include <algorithm>
 
 #include "sf_common.h"
